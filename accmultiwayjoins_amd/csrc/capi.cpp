@@ -1,4 +1,5 @@
 // extern "C" entry points of libamj (declared in include/amj.h).
+#include <algorithm>
 #include <cstring>
 
 #include "runtime.h"
@@ -100,6 +101,9 @@ int amj_ctx_create(int device, amj_ctx_t** out) {
     return AMJ_ERR_HIP;
   for (auto& e : ctx->ev)
     if (hipEventCreate(&e) != hipSuccess) return AMJ_ERR_HIP;
+  if (hipHostMalloc((void**)&ctx->mail, MAIL_WORDS * sizeof(uint64_t), hipHostMallocDefault) !=
+      hipSuccess)
+    return AMJ_ERR_HIP;
   *out = ctx.release();
   return AMJ_OK;
 }
@@ -113,6 +117,7 @@ void amj_ctx_destroy(amj_ctx_t* ctx) {
   if (ctx->arena.base) dfree(ctx, ctx->arena.base, ctx->arena.size);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
+  if (ctx->mail) (void)hipHostFree(ctx->mail);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   delete ctx;
@@ -219,6 +224,11 @@ void amj_hash_table_destroy(amj_ctx_t* ctx, amj_hash_table_t* ht) {
   dfree(ctx, ht->dev.ptrs, (ht->dev.buckets + 1) * 4);
   dfree(ctx, ht->dev.keys, n * 4);
   dfree(ctx, ht->dev.vals, n * 4);
+  if (ht->dev.rec) {
+    const uint64_t rec = ht->dev.buckets * sizeof(uint4);
+    dfree(ctx, ht->dev.rec, rec);
+    if (ctx) ctx->rec_bytes -= std::min(ctx->rec_bytes, rec);
+  }
   delete ht;
 }
 

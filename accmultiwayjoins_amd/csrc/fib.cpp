@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "colsort.h"
 #include "runtime.h"
 
 namespace amj {
@@ -77,18 +78,24 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
     for (int c = 0; c < P.probe_ncols; ++c)
       if (P.probe_attr[c] == P.key_attr[0]) kcol = c;
     const int other = P.probe_ncols == 2 ? 1 - kcol : -1;
-    void *comp = nullptr, *alt = nullptr, *tmp = nullptr, *cols = nullptr;
-    AMJ_TRY(scratch(ctx, SLOT_SORT_KEYS, np * 8, &comp));
-    AMJ_TRY(scratch(ctx, SLOT_SORT_ALT, np * 8, &alt));
-    AMJ_TRY(scratch(ctx, SLOT_SORT_TEMP, radix_sort_temp_bytes(np), &tmp));
+    void *x = nullptr, *y = nullptr, *tmp = nullptr, *cols = nullptr;
+    AMJ_TRY(scratch(ctx, SLOT_SORT_KEYS, np * 8, &x));
+    AMJ_TRY(scratch(ctx, SLOT_SORT_ALT, np * 8, &y));
+    AMJ_TRY(scratch(ctx, SLOT_SORT_TEMP, col_sort_temp_bytes(np), &tmp));
     AMJ_TRY(scratch(ctx, SLOT_PROBE_SORTED, np * 4 * P.probe_ncols, &cols));
     int32_t* sk = (int32_t*)cols;
     int32_t* so = other >= 0 ? sk + np : nullptr;
-    AMJ_HIP_TRY(ctx, launch_pack_composite(P.probe_cols[kcol],
-                                           other >= 0 ? P.probe_cols[other] : nullptr, np, 0,
-                                           (uint64_t*)comp, s));
-    AMJ_HIP_TRY(ctx, radix_sort_u64((uint64_t*)comp, (uint64_t*)alt, np, 0xf0u, tmp, s));
-    AMJ_HIP_TRY(ctx, launch_unpack_composite((const uint64_t*)comp, np, 0, sk, so, s));
+    ColSort c;
+    c.key = P.probe_cols[kcol];
+    c.val = other >= 0 ? P.probe_cols[other] : nullptr;
+    c.n = np;
+    c.mask = 0xf0u;
+    c.buf_x = (uint64_t*)x;
+    c.buf_y = (uint64_t*)y;
+    c.out_key = sk;
+    c.out_val = so;
+    ColSortFacts facts;
+    AMJ_HIP_TRY(ctx, run_col_sort(c, tmp, ctx->mail + MAIL_SORT, ctx->ev[6], s, &facts));
     P.probe_cols[kcol] = sk;
     if (other >= 0) P.probe_cols[other] = so;
   }

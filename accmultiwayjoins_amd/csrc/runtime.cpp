@@ -1,5 +1,6 @@
 // Host runtime of libamj: context, device buffers, relations, hash build driver, query
 // planning and the AMHJ execution driver (count/scan/write and frequent-item paths).
+#include "colsort.h"
 #include "runtime.h"
 #include "tpt.h"
 
@@ -78,6 +79,18 @@ int scratch(amj_ctx_t* ctx, int slot, size_t bytes, void** out) {
 // ------------------------------------------------------------------------------------------
 // Hash build.
 // ------------------------------------------------------------------------------------------
+// Bucket records of a table (16 B per bucket), left out (d->rec == nullptr) when they would bring
+// the context's records over an eighth of the device memory or cannot be allocated.
+static int alloc_records(amj_ctx_t* ctx, HashTableDev* d) {
+  const uint64_t bytes = d->buckets * sizeof(uint4);
+  d->rec = nullptr;
+  if (bytes > (1ull << 20) && ctx->rec_bytes + bytes > (uint64_t)ctx->props.totalGlobalMem / 8)
+    return AMJ_OK;
+  if (dmalloc(ctx, (void**)&d->rec, bytes) == AMJ_OK) ctx->rec_bytes += bytes;
+  else d->rec = nullptr;
+  return AMJ_OK;
+}
+
 int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, int sort_vals,
                      amj_hash_table** out) {
   *out = nullptr;
@@ -107,12 +120,6 @@ int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, 
 
   hipStream_t s = ctx->stream;
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[0], s));
-  void *comp = nullptr, *alt = nullptr, *tmp = nullptr, *flag = nullptr;
-  AMJ_TRY(scratch(ctx, SLOT_SORT_KEYS, std::max<uint64_t>(n, 1) * 8, &comp));
-  AMJ_TRY(scratch(ctx, SLOT_SORT_ALT, std::max<uint64_t>(n, 1) * 8, &alt));
-  AMJ_TRY(scratch(ctx, SLOT_SORT_TEMP, radix_sort_temp_bytes(std::max<uint64_t>(n, 1)), &tmp));
-  AMJ_TRY(scratch(ctx, SLOT_FLAG, 256, &flag));
-
   auto& d = ht->dev;
   d.buckets = buckets;
   AMJ_TRY(dmalloc(ctx, (void**)&d.ptrs, (buckets + 1) * sizeof(uint32_t)));
@@ -121,28 +128,55 @@ int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, 
 
   uint32_t identity = 0;
   if (n > 0) {
-    AMJ_HIP_TRY(ctx, launch_pack_composite(key, val, n, log_b, (uint64_t*)comp, s));
+    ColSort c;
+    c.key = key;
+    c.val = val;
+    c.n = n;
+    c.rot = log_b;
     // sort digits 4..7 (hash column) always, 0..3 (second column) when it is compared
-    const uint32_t mask = sort_vals && val ? 0xffu : 0xf0u;
-    AMJ_HIP_TRY(ctx, radix_sort_u64((uint64_t*)comp, (uint64_t*)alt, n, mask, tmp, s));
-    AMJ_HIP_TRY(ctx, launch_unpack_composite((const uint64_t*)comp, n, log_b, d.keys, d.vals, s));
-    AMJ_HIP_TRY(ctx, launch_bucket_ptrs((const uint64_t*)comp, n, log_b, buckets, d.ptrs, s));
-    AMJ_HIP_TRY(ctx, launch_key_range(key, n, log_b, (uint32_t*)flag, s));
-    uint32_t hflag = 1;
-    AMJ_HIP_TRY(ctx, hipMemcpyAsync(&hflag, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
-    identity = hflag == 0 ? 1u : 0u;
+    c.mask = sort_vals && val ? 0xffu : 0xf0u;
+    c.key_limit = (uint32_t)buckets;
+    c.out_key = d.keys;
+    c.out_val = d.vals;
+    if (n <= kHashSmallRows) {
+      uint32_t* flag = (uint32_t*)(ctx->mail + MAIL_KEY_RANGE);
+      AMJ_TRY(alloc_records(ctx, &d));
+      if (!d.rec) {
+        set_error(ctx, AMJ_ERR_NOMEM, "no device memory for the bucket records");
+        return AMJ_ERR_NOMEM;
+      }
+      AMJ_HIP_TRY(ctx, launch_hash_small(c, log_b, d.ptrs, d.rec, flag, s));
+      AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[1], s));
+      AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[1]));
+      identity = *(volatile uint32_t*)flag == 0 ? 1u : 0u;
+    } else {
+      void *x = nullptr, *y = nullptr, *tmp = nullptr;
+      AMJ_TRY(scratch(ctx, SLOT_SORT_KEYS, n * 8, &x));
+      AMJ_TRY(scratch(ctx, SLOT_SORT_ALT, n * 8, &y));
+      AMJ_TRY(scratch(ctx, SLOT_SORT_TEMP, col_sort_temp_bytes(n), &tmp));
+      c.buf_x = (uint64_t*)x;
+      c.buf_y = (uint64_t*)y;
+      ColSortFacts facts;
+      AMJ_HIP_TRY(ctx, run_col_sort(c, tmp, ctx->mail + MAIL_SORT, ctx->ev[6], s, &facts));
+      // known while the device sorts: only tables that are not "identity" have records
+      identity = facts.past_limit ? 0u : 1u;
+      if (!identity) AMJ_TRY(alloc_records(ctx, &d));
+      AMJ_HIP_TRY(ctx, launch_bucket_index(d.keys, n, buckets, d.ptrs, d.rec, s));
+      AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[1], s));
+      AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[1]));
+    }
   } else {
     AMJ_HIP_TRY(ctx, hipMemsetAsync(d.ptrs, 0, (buckets + 1) * sizeof(uint32_t), s));
+    AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[1], s));
+    AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[1]));
   }
-  AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[1], s));
-  AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[1]));
   ht->build_ms = elapsed_ms(ctx->ev[0], ctx->ev[1]);
 
   d.view.ptrs = d.ptrs;
   d.view.keys = d.keys;
   d.view.vals = d.vals;
   d.view.pw = nullptr;
+  d.view.rec = identity ? nullptr : d.rec;
   d.view.n = n;
   d.view.log_b = log_b;
   d.view.identity = identity;
@@ -443,7 +477,8 @@ uint64_t budget_left(amj_ctx_t* ctx, const amj_opts_t* o) {
   uint64_t left = free_b + ctx->pool_bytes;  // parked buffers are reusable
   if (ctx->arena.base) left = arena_largest(ctx);
   if (o && o->hbm_budget_bytes) {
-    const uint64_t cap = o->hbm_budget_bytes > ctx->allocated ? o->hbm_budget_bytes - ctx->allocated : 0;
+    const uint64_t held = budget_held(ctx);
+    const uint64_t cap = o->hbm_budget_bytes > held ? o->hbm_budget_bytes - held : 0;
     left = std::min<uint64_t>(left, cap);
   }
   return left;

@@ -11,6 +11,9 @@ constexpr int kMaxLftjRels = 6;   // the 4-clique query joins six relations
 // Two-level sorted trie of a relation R(x, y) (IndexedTrie<D,C> with 2 attributes,
 // LFTJ-GPU/IndexedTrie.cuh:21-54): d0 = distinct x ascending, off[j] .. off[j+1] the children of
 // d0[j] in d1 (ascending, distinct).
+// Every child array on the device is followed by this many readable values, so that a wave may
+// load a batch that reaches past the last list without testing for it.
+constexpr uint64_t kTriePad = 256;
 struct LRel {
   const int32_t* d0;
   const uint32_t* off;  // [n0 + 1]
@@ -28,6 +31,7 @@ struct TrieDev {
   uint2* vrange = nullptr;
   uint32_t n0 = 0, n1 = 0, vrange_n = 0;
   uint32_t max_run = 0;  // longest child list
+  bool distinct = false;  // no child list holds a value twice
   double build_ms = 0.0;
 };
 
@@ -45,7 +49,7 @@ struct LPlan {
   int32_t off32;                       // every trie array is addressable with 32-bit byte offsets
   uint64_t roots;                      // level-0 size of driver0
   uint32_t rpu;                        // roots per unit of the DFS (1..64; 0: 64)
-  uint32_t pad;
+  uint32_t distinct;                   // no child list holds a value twice
 };
 
 // Query shapes with kernels of their own: relations listed by (x, y) ascending (the order the

@@ -46,20 +46,44 @@ __device__ __forceinline__ void level0(const LPlan& P, uint64_t unit, LLv<A>& l)
   level0_at<A, SH>(P, r, lane < rpu && r < P.roots, l);
 }
 
+// Result hash in two parts (hash_tuple: one round per pair of attributes): the first pair's round,
+// which all results of one entry share, and the rest.
+template <int A>
+__device__ __forceinline__ uint64_t hash_first_pair(int32_t b0, int32_t b1) {
+  return mix64((uint64_t)A ^ ((uint64_t)(uint32_t)b0 | ((uint64_t)(uint32_t)b1 << 32)));
+}
+template <int A>
+__device__ __forceinline__ uint64_t hash_rest(uint64_t h, const int32_t (&b)[A]) {
+  static_assert(A == 3 || A == 4, "one round after the first pair");
+  uint64_t w = (uint32_t)b[2];
+  if constexpr (A == 4) w |= (uint64_t)(uint32_t)b[3] << 32;
+  return mix64(h ^ w);
+}
+
 // What happens to the candidates that pass the last attribute (`ok` per lane, bindings in b):
-// counted, written at their scanned positions, or gathered for direct output.
+// counted, written at their scanned positions, or gathered for direct output. put() is the same
+// with the hash of the first pair given (kHashes sinks only look at it).
 struct CountSink {
+  static constexpr bool kCounts = true;  // add() is enough: the bindings are not looked at
+  static constexpr bool kHashes = false, kStores = false;
   uint64_t count = 0;
+  __device__ __forceinline__ void add(uint32_t n) { count += n; }
   template <int A>
   __device__ __forceinline__ void operator()(bool ok, const int32_t (&)[A]) {
     count += (uint64_t)__popcll(__ballot(ok));
+  }
+  template <int A>
+  __device__ __forceinline__ void put(bool ok, const int32_t (&b)[A], uint64_t) {
+    (*this)(ok, b);
   }
 };
 
 // Count and checksum only (the work-sharing engine's passes without output).
 template <bool HASH>
 struct CountHashSink {
+  static constexpr bool kCounts = !HASH, kHashes = HASH, kStores = false;
   uint64_t count = 0;
+  __device__ __forceinline__ void add(uint32_t n) { count += n; }
   uint64_t csum = 0;  // per-lane checksum partial
   template <int A>
   __device__ __forceinline__ void operator()(bool ok, const int32_t (&b)[A]) {
@@ -70,10 +94,16 @@ struct CountHashSink {
       csum += hash_tuple(w, A);
     }
   }
+  template <int A>
+  __device__ __forceinline__ void put(bool ok, const int32_t (&b)[A], uint64_t h) {
+    count += (uint64_t)__popcll(__ballot(ok));
+    if (HASH && ok) csum += hash_rest<A>(h, b);
+  }
 };
 
 template <int MODE>
 struct WriteSink {
+  static constexpr bool kCounts = false, kHashes = mode_hash<MODE>(), kStores = mode_mat<MODE>();
   LOut cols;
   uint64_t out_base;  // absolute row of the next result (uniform)
   uint64_t csum;      // per-lane checksum partial
@@ -86,6 +116,18 @@ struct WriteSink {
         sfor<0, kMaxAttrs>([&](auto a) { w[a] = (a < A) ? b[(a < A) ? (int)a : 0] : 0; });
         csum += hash_tuple(w, A);
       }
+      if (mode_mat<MODE>()) {
+        const uint64_t pos = out_base + mbcnt(m);
+        sfor<0, A>([&](auto a) { cols.c[a][pos] = b[a]; });
+      }
+    }
+    out_base += (uint64_t)__popcll(m);
+  }
+  template <int A>
+  __device__ __forceinline__ void put(bool ok, const int32_t (&b)[A], uint64_t h) {
+    const uint64_t m = __ballot(ok);
+    if (ok) {
+      if (mode_hash<MODE>()) csum += hash_rest<A>(h, b);
       if (mode_mat<MODE>()) {
         const uint64_t pos = out_base + mbcnt(m);
         sfor<0, A>([&](auto a) { cols.c[a][pos] = b[a]; });
@@ -112,6 +154,7 @@ typedef __attribute__((address_space(3))) int32_t lds_i32;
 // per result on the lanes whose candidate passed.
 template <int A, bool HASH>
 struct DirectSink {
+  static constexpr bool kCounts = false, kHashes = false, kStores = true;  // hashes when it flushes
   LOut cols;
   uint64_t capacity;
   unsigned long long* rows;  // rows reserved by the whole launch
@@ -186,6 +229,7 @@ struct DirectSink {
     __asm__ __volatile__("" ::: "memory");
     fill += n;
   }
+  __device__ __forceinline__ void put(bool ok, const int32_t (&b)[A], uint64_t) { (*this)(ok, b); }
 };
 
 // Candidates [c, c + 64) of the flattened level `par` (those below `end` are valid) checked
@@ -217,21 +261,27 @@ __device__ __forceinline__ bool lchild(const LPlan& P, const LLv<A>& par, uint32
   return ok;
 }
 
-// Last attribute of a compiled shape. An entry whose driver list holds at least
-// kCoopMinCands candidates and whose other child lists (every child list of the attribute but
-// the driver's) hold at most kStageInts values together is run by the whole wave: the other
-// lists are copied to the wave's LDS stage once, and each chunk of 64 candidates is checked
-// there by binary searches of uniform length (one global load per candidate instead of a
-// chain of dependent ones). The other entries go through the flattened enumeration.
+// Cooperative levels of the compiled shapes: entries whose lists are long enough are run by the
+// whole wave, which keeps the values of one list in LDS and checks the other list's values
+// against them; the rest go through the flattened enumeration.
 constexpr uint32_t kCoopMinCands = 32;
-constexpr uint32_t kStageInts = 1024;  // per wave
-// 4-clique pairs (descend_clique_pairs): the other list of an entry (at most kCliqueOther
-// values) and the entry's intersection after it, in a stage of 2 * kCliqueOther values.
+constexpr uint32_t kStageInts = 1024;  // values of the checked list, at most
+// 4-clique pairs (descend_clique_pairs): the checked list of an entry, and the entry's
+// intersection.
 constexpr uint32_t kCliqueOther = 768;
+// LDS words per wave: the kept list's table (or, in a list no table could be made of, its values),
+// and the queue of results. 4-cliques have besides the entry's intersection and its table. Sized
+// so that four workgroups (4-cliques: three) fit a CU.
+constexpr uint32_t kTriTable = 2048, kFourTable = 1024, kPairTable = 1024;
+constexpr uint32_t kQueue = 128;                               // results: a word and a byte each
+constexpr uint32_t kQueueWords = kQueue + kQueue / 4;
 template <uint64_t SH>
 constexpr uint32_t stage_ints() {
-  return SH == kShapeFour ? 2 * kCliqueOther : kStageInts;
+  return SH == kShapeFour ? kFourTable + kCliqueOther + kPairTable + kQueueWords
+                          : kTriTable + kQueueWords;
 }
+static_assert(kStageInts <= kTriTable && kCliqueOther <= kFourTable, "a list fits its table's room");
+static_assert(kStageInts <= kFourTable, "descend_last_fixed stages into the 4-clique's table");
 
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
@@ -271,6 +321,273 @@ __device__ __forceinline__ void lds_has(const lds_i32* st, uint32_t n, const int
 // Chunks of 64 candidates a wave checks at once in the cooperative last level.
 constexpr int kCoopChunks = 4;
 
+// The values of an ascending list, kept in LDS for membership tests: a cuckoo table (every value in
+// one of its two slots, so a test is two independent reads), at most 7/16 full; or, when the list
+// is too long for the room or the insertion does not settle (values that share their slots), the
+// list itself, searched.
+//
+// An empty slot s holds s ^ 1, which no test of that slot can match: the first hash of s ^ 1 is
+// s ^ 1 (values below 2^11 hash to themselves), and kHashMul was chosen so that its second hash is
+// not s either, for every slot of every table size from 64 to 2,048.
+constexpr uint32_t kHashMul = 0x9ad2d5u;
+struct LdsSet {
+  lds_i32* t;          // table or list
+  uint32_t n = 0;      // values
+  uint32_t m4 = 0;     // byte mask of a slot's offset (0: t is the list)
+
+  static __device__ __forceinline__ uint32_t mix(int32_t v) {
+    return (uint32_t)v ^ ((uint32_t)v >> 11);
+  }
+  __device__ __forceinline__ uint32_t slot1(uint32_t x) const { return (x << 2) & m4; }
+  __device__ __forceinline__ uint32_t slot2(uint32_t x) const {
+    return (__umul24(x, kHashMul) >> 10) & m4;
+  }
+  __device__ __forceinline__ lds_i32* at(uint32_t off) const {
+    return (lds_i32*)((__attribute__((address_space(3))) char*)t + off);
+  }
+  // load(i): value i of the list, i < n_values (n_values > 0); `room` words at t
+  template <typename Load>
+  __device__ __forceinline__ void fill(uint32_t n_values, uint32_t room, Load&& load) {
+    const uint32_t lane = (uint32_t)lane_id();
+    __asm__ __volatile__("" ::: "memory");  // LDS ops of one wave complete in order
+    n = n_values;
+    uint32_t words = (uint32_t)kWave;
+    while (words < room && words < 4 * n_values) words <<= 1;
+    bool settled = 16 * n_values <= 7 * words;
+    if (settled) {
+      m4 = (words - 1) << 2;
+      for (uint32_t i = lane; i < words; i += kWave) t[i] = (int32_t)(i ^ 1u);
+      __asm__ __volatile__("" ::: "memory");
+      for (uint32_t j0 = 0; j0 < n_values && settled; j0 += kWave) {
+        bool todo = j0 + lane < n_values;
+        int32_t v = load(todo ? j0 + lane : n_values - 1);
+        uint32_t off = slot1(mix(v));
+        int left = 48;  // rounds of evictions
+        for (; left && __ballot(todo); --left) {
+          if (todo) {
+            const int32_t old = __hip_atomic_exchange(at(off), v, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_WAVEFRONT);
+            todo = (uint32_t)old != ((off >> 2) ^ 1u);
+            v = old;
+            const uint32_t x = mix(old), o1 = slot1(x);
+            off = o1 == off ? slot2(x) : o1;
+          }
+        }
+        settled = __ballot(todo) == 0ull;
+      }
+    }
+    if (!settled) {
+      m4 = 0;
+      __asm__ __volatile__("" ::: "memory");
+      for (uint32_t j = lane; j < n_values; j += kWave) t[j] = load(j);
+    }
+    __asm__ __volatile__("" ::: "memory");
+  }
+  // live[j] loses the lanes whose v[j] is not in the list
+  template <int K>
+  __device__ __forceinline__ void keep(const int32_t (&v)[K], uint64_t (&live)[K]) const {
+    if (m4) {
+      int32_t a[K], b[K];  // all reads in flight together
+      sfor<0, K>([&](auto j) {
+        const uint32_t x = mix(v[j]);
+        a[j] = *at(slot1(x));
+        b[j] = *at(slot2(x));
+      });
+      sfor<0, K>([&](auto j) { live[j] &= __ballot(a[j] == v[j]) | __ballot(b[j] == v[j]); });
+    } else {
+      bool ok[K];
+      sfor<0, K>([&](auto j) { ok[j] = true; });
+      lds_has<K>(t, n, v, ok);
+      sfor<0, K>([&](auto j) { live[j] &= __ballot(ok[j]); });
+    }
+  }
+};
+
+// Results gathered to full waves, in the order they came: a ring of (value, tag < 64) pairs.
+struct Hits {
+  lds_i32* ring;
+  uint32_t head = 0, n = 0;  // uniform
+
+  __device__ __forceinline__ __attribute__((address_space(3))) uint8_t* tags() const {
+    return (__attribute__((address_space(3))) uint8_t*)(ring + kQueue);
+  }
+  __device__ __forceinline__ void push(uint64_t m, int32_t v, int tag) {
+    if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+      const uint32_t at = (head + n + mbcnt(m)) & (kQueue - 1);
+      ring[at] = v;
+      tags()[at] = (uint8_t)tag;
+    }
+    n += (uint32_t)__popcll(m);
+  }
+  // Takes the first min(n, 64): f(valid, value, tag).
+  template <typename F>
+  __device__ __forceinline__ void take(F&& f) {
+    const uint32_t lane = (uint32_t)lane_id();
+    const uint32_t k = n < (uint32_t)kWave ? n : (uint32_t)kWave;
+    __asm__ __volatile__("" ::: "memory");  // LDS ops of one wave complete in order
+    const uint32_t at = (head + lane) & (kQueue - 1);
+    const int32_t v = ring[at];
+    const int tag = (int)tags()[at] & (kWave - 1);
+    head += k;
+    n -= k;
+    __asm__ __volatile__("" ::: "memory");
+    f(lane < k, v, tag);
+  }
+};
+
+// The lists of the entries in `m` (lane p's list: ptr, len > 0, in a child array with kTriePad
+// readable values after its end), one after the other, kStream x 64 values at a time: enter(p)
+// before an entry's values, then step(v, live, p), v[j] being the values of chunk j, live[j] its
+// lanes that hold one (0: chunk not there). The next values, of the same list or the next entry's,
+// are loaded before the current ones are taken; the loads have neither conditions nor address
+// arithmetic per lane.
+constexpr int kStream = 4;
+static_assert(kStream * kWave <= (int)kTriePad, "a batch may be read past the end of a list");
+template <typename Enter, typename Step>
+__device__ __forceinline__ void stream_lists(uint64_t m, const int32_t* ptr, uint32_t len,
+                                             Enter&& enter, Step&& step) {
+  if (m == 0) return;
+  constexpr uint32_t kTake = (uint32_t)(kStream * kWave);
+  const uint32_t lane = (uint32_t)lane_id();
+  const auto fetch = [&](const int32_t* q, int32_t (&v)[kStream]) {
+    typedef __attribute__((address_space(1))) const char gchar;
+    uint32_t off = lane * 4u;
+    __asm__("" : "+v"(off));  // kept a 32-bit offset from the uniform q, not a 64-bit address
+    const gchar* at = (const gchar*)q + off;
+    sfor<0, kStream>([&](auto j) {
+      v[j] = *(__attribute__((address_space(1))) const int32_t*)(at + (int)j * 4 * kWave);
+    });
+  };
+  int p = __ffsll((unsigned long long)m) - 1;
+  const int32_t* q = (const int32_t*)readlane_u64((uint64_t)ptr, p);
+  uint32_t l = readlane_u32(len, p);
+  int32_t v[kStream];
+  fetch(q, v);
+  for (;;) {
+    m &= m - 1;
+    const int pn = m ? __ffsll((unsigned long long)m) - 1 : p;
+    const int32_t* qn = (const int32_t*)readlane_u64((uint64_t)ptr, pn);
+    const uint32_t ln = readlane_u32(len, pn);
+    enter(p);
+    for (;;) {
+      int32_t w[kStream];
+      const bool more = l > kTake;
+      q = more ? q + kTake : qn;
+      fetch(q, w);
+      uint64_t live[kStream];
+      sfor<0, kStream>([&](auto j) { live[j] = __ballot(lane + (uint32_t)j * kWave < l); });
+      step(v, live, p);
+      sfor<0, kStream>([&](auto j) { v[j] = w[j]; });
+      if (!more) break;
+      l -= kTake;
+    }
+    if (!m) break;
+    p = pn;
+    l = ln;
+  }
+}
+
+// Lists of this many values on average are streamed one by one, shorter ones flattened over the
+// wave: a list pays for whole chunks of 64, a flattened chunk for finding every value's list.
+constexpr uint32_t kStreamMean = 96;
+
+// Which of an entry's two child lists is checked against and which is streamed. With lists free of
+// duplicates that are whole (not cut to a window of candidates) the first relation's list is
+// kept in LDS and the second one's streamed: consecutive entries share their first value, so
+// the kept list and its bitmap stay. Otherwise the candidates' own list is streamed, which is what
+// decides how often a duplicate is produced.
+template <int A>
+struct PairLists {
+  const int32_t *set, *str;
+  uint32_t set_n, str_n;
+  __device__ __forceinline__ PairLists(const LPlan& P, const LLv<A>& l, int ra, int rb) {
+    const int32_t* pa = P.rel[ra].d1 + l.lo[ra];
+    const int32_t* pb = P.rel[rb].d1 + l.lo[rb];
+    const uint32_t na = l.hi[ra] - l.lo[ra], nb = l.hi[rb] - l.lo[rb];
+    const bool drives_b = l.drel == rb;
+    const bool whole = l.dlen == (drives_b ? nb : na);
+    const bool stream_b = drives_b || (P.distinct && whole);
+    set = stream_b ? pa : pb;
+    set_n = stream_b ? na : nb;
+    str = drives_b || !stream_b ? l.dptr : pb;
+    str_n = drives_b || !stream_b ? l.dlen : nb;
+  }
+};
+
+// Last attribute of a triangle (compiled shape kShapeTri): a2 in the children of a0 (relation 1)
+// and of a1 (relation 2). Entries with at least kCoopMinCands candidates whose lists both fit the
+// stage are run by the whole wave: the children of a0 stay in LDS (a table) while the children of
+// every a1 are streamed past them, two independent LDS reads per value; the results (one value in
+// eleven on R-MAT 22) are gathered to full waves. They come in entry order, ascending.
+//
+// Bound by the streamed loads (23.8 G values for R-MAT 22) and about 15 VALU instructions per 64 of
+// them. The version before staged the longer list of every entry and searched the shorter one in
+// it (26 G values staged, 11.6 G searched in 9 to 10 steps), and its sinks saw the one in six
+// lanes that passed. R-MAT 22, count / write with checksum: 31.8 / 43.9 ms before, 27.6 / 35 ms now
+// (880 M lines of 128 B fetched past the L2 per pass, 4.2 TB/s); R-MAT 20, count with checksum 5.6
+// -> 4.6 ms.
+template <int A, uint64_t SH, typename Sink>
+__device__ __forceinline__ void descend_tri_last(const LPlan& P, const LLv<A>& par, Sink& sink,
+                                                 lds_i32* stage) {
+  static_assert(A == 3 && SH == kShapeTri, "triangle shape only");
+  const uint32_t na = par.hi[1] - par.lo[1], nb = par.hi[2] - par.lo[2];
+  const bool coop = par.dlen >= kCoopMinCands && (par.drel == 1 ? nb : na) <= kStageInts;
+  {  // entries with few candidates (or a long list to check): flattened
+    LLv<A> sm = par;
+    sm.dlen = coop ? 0u : par.dlen;
+    finish(sm);
+    for (uint32_t c = 0; c < sm.T; c += (uint32_t)kWave) {
+      LLv<A> ch;
+      const bool ok = lchild<A, 2, SH>(P, sm, c, sm.T, ch);
+      sink(ok, ch.b);
+    }
+  }
+  const PairLists<A> pl(P, par, 1, 2);
+  LdsSet set;
+  set.t = stage;
+  Hits hits;
+  hits.ring = stage + kTriTable;
+  const uint64_t h01 = Sink::kHashes ? hash_first_pair<A>(par.b[0], par.b[1]) : 0ull;
+  const auto emit = [&]() {
+    hits.take([&](bool ok, int32_t v, int p) {
+      int32_t b[A] = {0, 0, v};
+      if constexpr (Sink::kStores) {
+        b[0] = __shfl(par.b[0], p, kWave);
+        b[1] = __shfl(par.b[1], p, kWave);
+      }
+      sink.put(ok, b, Sink::kHashes ? __shfl(h01, p, kWave) : 0ull);
+    });
+  };
+  uint64_t kept = 0;
+  stream_lists(
+      __ballot(coop), pl.str, pl.str_n,
+      [&](int p) {
+        const uint64_t src = readlane_u64((uint64_t)pl.set, p);
+        const uint32_t n = readlane_u32(pl.set_n, p);
+        if (src == kept && n == set.n) return;
+        kept = src;
+        set.fill(n, kTriTable, [&](uint32_t i) { return ld_at<true>((const int32_t*)src, i); });
+      },
+      [&](const int32_t (&v)[kStream], uint64_t (&live)[kStream], int p) {
+        set.keep(v, live);
+        sfor<0, kStream>([&](auto j) {
+          if constexpr (Sink::kCounts) {
+            sink.add((uint32_t)__popcll(live[j]));
+          } else if (live[j]) {
+            hits.push(live[j], v[j], p);
+            if (hits.n >= (uint32_t)kWave) emit();
+          }
+        });
+      });
+  while (hits.n) emit();
+}
+
+// The last attribute of a 4-clique outside the clique pairs. An entry whose driver list holds at
+// least kCoopMinCands candidates and whose other child lists (every child list of the attribute
+// but the driver's) hold at most kStageInts values together is run by the whole wave: the other
+// lists are copied to the wave's LDS stage once, and each chunk of 64 candidates is checked
+// there by binary searches of uniform length (one global load per candidate instead of a
+// chain of dependent ones). The other entries go through the flattened enumeration.
 template <int A, int I, uint64_t SH, typename Sink>
 __device__ __forceinline__ void descend_last_fixed(const LPlan& P, const LLv<A>& par, Sink& sink,
                                                    lds_i32* stage) {
@@ -383,22 +700,22 @@ __device__ __forceinline__ void descend_last_fixed(const LPlan& P, const LLv<A>&
 // Attributes 2 and 3 of a 4-clique (compiled shape kShapeFour) whose relations (0,2) and (0,3)
 // are one trie, and (1,2) and (1,3) another. For an entry (a0, a1) the third attribute takes
 // L = children(a0) ∩ children'(a1), and the fourth takes the same L intersected with the children
-// of a2 in relation (2,3). An entry whose list to check holds at most kCliqueOther values is run
-// by the whole wave: L is formed once in LDS (the other list staged, the driver's candidates
-// checked there and the passing ones appended in order, so L stays sorted), then every a2 of L
-// opens its children in (2,3), and each child found in L is a result: one LDS search in the
-// short list L per candidate, instead of two searches in long lists per candidate. The other
-// entries take the generic path.
+// of a2 in relation (2,3). An entry whose lists hold at most kCliqueOther values is run by the
+// whole wave: L is formed once (the children of a1 streamed past those of a0, kept in LDS; the
+// values found appended in order), L gets a table of its own, and every child of every a2 of L is
+// one test in it (two LDS reads). The other entries take the generic path.
+//
+// Bound by issue and LDS latency: the table of L (up to 448 values) decides how many workgroups
+// fit a CU; one of a quarter of the size, with a fourth workgroup per CU, was slower (R-MAT 18 dense
+// cores have longer L: 72 ms against 44). Searching L instead, chunks flattened over the wave:
+// R-MAT 18 / 20 62 / 298 ms (unit engine, count + checksum), now 44 / 174 ms.
 template <int A, uint64_t SH, typename Sink>
 __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A>& par,
                                                      Sink& sink, lds_i32* stage) {
   static_assert(A == 4 && SH == kShapeFour, "4-clique shape only");
   constexpr int K = kCoopChunks;
-  // the relation checked at attribute 2 besides the driver (1: children of a0, 3: of a1)
-  const bool drv1 = par.drel == 1;
-  const int32_t* optr = drv1 ? P.rel[3].d1 + par.lo[3] : P.rel[1].d1 + par.lo[1];
-  const uint32_t olen = drv1 ? par.hi[3] - par.lo[3] : par.hi[1] - par.lo[1];
-  const bool clique = par.dlen > 0 && olen <= kCliqueOther;
+  const uint32_t na = par.hi[1] - par.lo[1], nb = par.hi[3] - par.lo[3];
+  const bool clique = par.dlen > 0 && na <= kCliqueOther && (par.drel == 1 ? nb : na) <= kCliqueOther;
 
   // entries with a long list to check: the generic levels
   {
@@ -414,91 +731,105 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
     }
   }
 
-  lds_i32* lst = stage + kCliqueOther;  // L
+  const PairLists<A> pl(P, par, 1, 3);
+  LdsSet set, pair;  // the kept list; L
+  set.t = stage;
+  lds_i32* lst = stage + kFourTable;  // L, ascending
+  pair.t = lst + kCliqueOther;
+  Hits hits;
+  hits.ring = pair.t + kPairTable;
+  uint64_t kept = 0;
   uint64_t m = __ballot(clique);
   const uint32_t lane = (uint32_t)lane_id();
-  uint64_t staged = 0;
-  uint32_t slen = 0;
   const LRel& r5 = P.rel[5];
   while (m) {
     const int p = __ffsll((unsigned long long)m) - 1;
     m &= m - 1;
-    const int32_t* dp = (const int32_t*)readlane_u64((uint64_t)par.dptr, p);
-    const uint32_t dl = readlane_u32(par.dlen, p);
-    const int32_t* src = (const int32_t*)readlane_u64((uint64_t)optr, p);
-    const uint32_t n = readlane_u32(olen, p);
-    if ((uint64_t)src != staged || n != slen) {
-      __asm__ __volatile__("" ::: "memory");  // earlier reads of the stage are done (in order)
-      for (uint32_t j0 = 0; j0 < n; j0 += 4u * kWave) {
-        int32_t t[4];
-        sfor<0, 4>([&](auto u) {
-          const uint32_t j = j0 + (uint32_t)u * kWave + lane;
-          t[u] = j < n ? ld_at<false>(src, j) : 0;
-        });
-        sfor<0, 4>([&](auto u) {
-          const uint32_t j = j0 + (uint32_t)u * kWave + lane;
-          if (j < n) stage[j] = t[u];
-        });
-      }
-      staged = (uint64_t)src;
-      slen = n;
-      __asm__ __volatile__("" ::: "memory");  // LDS ops of one wave complete in order
+    const uint64_t src = readlane_u64((uint64_t)pl.set, p);
+    const uint32_t n = readlane_u32(pl.set_n, p);
+    if (src != kept || n != set.n) {
+      kept = src;
+      set.fill(n, kFourTable, [&](uint32_t i) { return ld_at<true>((const int32_t*)src, i); });
     }
-    // L = the driver's candidates found in the staged list, in order
+    // L = the streamed values found in the kept list, in order
     uint32_t nl = 0;
-    for (uint32_t c = 0; c < dl; c += (uint32_t)(K * kWave)) {
-      int32_t v[K];
-      bool ok[K];
-      sfor<0, K>([&](auto j) {
-        const uint32_t g = c + (uint32_t)j * kWave + lane;
-        ok[j] = g < dl;
-        v[j] = ok[j] ? ld_at<false>(dp, g) : 0;
-      });
-      lds_has<K>(stage, n, v, ok);
-      sfor<0, K>([&](auto j) {
-        const uint64_t bm = __ballot(ok[j]);
-        if (ok[j]) lst[nl + mbcnt(bm)] = v[j];
-        nl += (uint32_t)__popcll(bm);
-      });
-    }
+    stream_lists(
+        1ull << p, pl.str, pl.str_n, [](int) {},
+        [&](const int32_t (&v)[kStream], uint64_t (&live)[kStream], int) {
+          set.keep(v, live);
+          sfor<0, kStream>([&](auto j) {
+            if (__builtin_amdgcn_inverse_ballot_w64(live[j])) lst[nl + mbcnt(live[j])] = v[j];
+            nl += (uint32_t)__popcll(live[j]);
+          });
+        });
     __asm__ __volatile__("" ::: "memory");
     if (nl == 0) continue;
     int32_t b[A];
     b[0] = (int32_t)readlane_u32((uint32_t)par.b[0], p);
     b[1] = (int32_t)readlane_u32((uint32_t)par.b[1], p);
-    // every a2 of L (64 at a time) with its children in (2,3), flattened over the wave
+    const uint64_t h01 = Sink::kHashes ? hash_first_pair<A>(b[0], b[1]) : 0ull;
+    // a list longer than the table's room is searched where it lies
+    if (nl <= kPairTable) {
+      pair.t = lst + kCliqueOther;
+      pair.fill(nl, kPairTable, [&](uint32_t i) { return lst[i]; });
+    } else {
+      pair.t = lst;
+      pair.n = nl;
+      pair.m4 = 0;
+    }
+    // every a2 of L (64 at a time), its children in (2,3) checked against L: streamed list by
+    // list, or, when the lists are short, flattened over the wave
     for (uint32_t g0 = 0; g0 < nl; g0 += (uint32_t)kWave) {
       const bool has = g0 + lane < nl;
       const int32_t a2 = has ? lst[g0 + lane] : 0;
       uint32_t clo = 0, chi = 0;
       const bool f = has && root_range<true>(r5, a2, clo, chi);
-      const uint32_t len = f ? chi - clo : 0u;
-      const uint32_t incl = wave_scan_add_dpp(len);
-      const uint32_t excl = incl - len;
+      const uint32_t clen = f ? chi - clo : 0u;
+      const uint32_t incl = wave_scan_add_dpp(clen);
       const uint32_t T = lane63(incl);
-      for (uint32_t c = 0; c < T; c += (uint32_t)(K * kWave)) {
-        // K chunks of 64 candidates at once: their loads and searches are in flight together
-        int q[K];
-        bool ok[K];
-        int32_t a3[K];
-        sfor<0, K>([&](auto j) {
-          const uint32_t cj = c + (uint32_t)j * kWave;
-          const uint32_t g = cj + lane;
-          q[j] = (int)parent_of_slots(excl, len, cj < T ? cj : 0u);
-          const uint32_t k = g - (uint32_t)__shfl(excl, q[j], kWave);
-          const uint32_t qlo = (uint32_t)__shfl(clo, q[j], kWave);
-          ok[j] = g < T;
-          a3[j] = ok[j] ? ld_at<false>(r5.d1, qlo + k) : 0;
+      const uint64_t fm = __ballot(f);
+      const auto emit = [&]() {
+        hits.take([&](bool ok, int32_t v, int q) {
+          b[2] = __shfl(a2, q, kWave);
+          b[3] = v;
+          sink.put(ok, b, h01);
         });
-        lds_has<K>(lst, nl, a3, ok);
-        sfor<0, K>([&](auto j) {
-          if (c + (uint32_t)j * kWave < T) {
-            b[2] = __shfl(a2, q[j], kWave);
-            b[3] = a3[j];
-            sink(ok[j], b);
-          }
-        });
+      };
+      const auto found = [&](uint64_t hit, int32_t v, int q) {
+        if constexpr (Sink::kCounts) {
+          sink.add((uint32_t)__popcll(hit));
+        } else if (hit) {
+          hits.push(hit, v, q);
+          if (hits.n >= (uint32_t)kWave) emit();
+        }
+      };
+      if (T >= kStreamMean * (uint32_t)__popcll(fm)) {
+        stream_lists(
+            fm, r5.d1 + clo, clen, [](int) {},
+            [&](const int32_t (&v)[kStream], uint64_t (&live)[kStream], int q) {
+              pair.keep(v, live);
+              sfor<0, kStream>([&](auto j) { found(live[j], v[j], q); });
+            });
+      } else {
+        const uint32_t excl = incl - clen;
+        for (uint32_t c = 0; c < T; c += (uint32_t)(K * kWave)) {
+          int q[K];
+          int32_t a3[K];
+          uint64_t live[K];
+          sfor<0, K>([&](auto j) {
+            const uint32_t cj = c + (uint32_t)j * kWave;
+            const uint32_t g = cj + lane;
+            q[j] = (int)parent_of_slots(excl, clen, cj < T ? cj : 0u);
+            const uint32_t k = g - (uint32_t)__shfl(excl, q[j], kWave);
+            const uint32_t qlo = (uint32_t)__shfl(clo, q[j], kWave);
+            live[j] = __ballot(g < T);
+            a3[j] = ld_at<true>(r5.d1, g < T ? qlo + k : clo);
+          });
+          pair.keep(a3, live);
+          sfor<0, K>([&](auto j) { found(live[j], a3[j], q[j]); });
+        }
       }
+      while (hits.n) emit();
     }
   }
 }
@@ -506,7 +837,9 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
 template <int A, int i, uint64_t SH = 0, typename Sink>
 __device__ __forceinline__ void descend(const LPlan& P, const LLv<A>& par, Sink& sink,
                                         lds_i32* stage = nullptr) {
-  if constexpr (SH != 0 && i == A - 1) {
+  if constexpr (SH == kShapeTri && i == A - 1) {
+    descend_tri_last<A, SH>(P, par, sink, stage);
+  } else if constexpr (SH != 0 && i == A - 1) {
     descend_last_fixed<A, i, SH>(P, par, sink, stage);
   } else if constexpr (SH == kShapeFour && i == 2) {
     // (0,2) and (0,3) one trie, (1,2) and (1,3) another: the clique pairs apply

@@ -46,6 +46,7 @@ static int make_lplan(amj_ctx_t* ctx, const std::vector<LUse>& uses, const uint3
   P->n_attrs = (int32_t)na;
   P->n_rels = (int32_t)uses.size();
   P->off32 = 1;
+  P->distinct = 1;
   uint64_t widest = 0;  // longest candidate list any frontier entry can take
   for (size_t r = 0; r < uses.size(); ++r) {
     const int px = pos_of(uses[r].x_id), py = pos_of(uses[r].y_id);
@@ -65,6 +66,7 @@ static int make_lplan(amj_ctx_t* ctx, const std::vector<LUse>& uses, const uint3
     P->child_mask[py] |= 1u << r;
     widest = std::max<uint64_t>(widest, uses[r].t->dev.max_run);
     const TrieDev& d = uses[r].t->dev;
+    if (!d.distinct) P->distinct = 0;
     if ((uint64_t)d.n0 + 1 >= (1ull << 30) || d.n1 >= (1ull << 30) || d.vrange_n >= (1u << 29))
       P->off32 = 0;
   }
@@ -291,6 +293,13 @@ static int run_lftj_count(amj_ctx_t* ctx, const LPlan& P, amj_result_t* res) {
 // output is sized by a counting pass (or, with dro, from the sample of the direct-output path)
 // and written in one pass with direct output; an overrun runs once more into an exact size.
 constexpr uint64_t kLftjSplit = 1024;        // ALFTJ.cuh:22 BUC_THRESHOLD
+// Compiled shapes (which share runs of their second attribute only) at the default split: a task
+// costs tens of microseconds of queue traffic and a claim tenths of one, so balance comes first from
+// small units claimed one at a time, heaviest first, and only runs far longer than a unit's
+// average are shared (a 4-clique's are worth more than a triangle's). R-MAT 18 / 20 with units of
+// 64 roots claimed several at a time and every run over 1,088 shared: triangles 13.9 / 32 ms,
+// 4-cliques 60 / 186 ms; so 2.2 / 5.5 ms and 45 / 185 ms.
+constexpr uint64_t kWsUnitsPerWave = 2;
 constexpr uint64_t kLftjTaskSlots = 8192;    // task records of 5,440 bytes
 constexpr uint64_t kLftjStallMs = 20000;     // no progress for this long: give up
 
@@ -317,15 +326,9 @@ static int lftj_ws_pass(amj_ctx_t* ctx, const LPlan& P, const LOut& out, int mod
 static int run_lftj_ws(amj_ctx_t* ctx, const LPlan& P_in, const amj_opts_t* o,
                        amj_result_t* res) {
   hipStream_t s = ctx->stream;
-  // units of 64 roots: the waves claim them dynamically and split long runs into tasks, so
-  // they need not be small
   LPlan P = P_in;
-  P.rpu = kWave;
-  const uint64_t units = lftj_units(P);
   WsArgs A{};
   void *ctl = nullptr, *tasks = nullptr, *ready = nullptr;
-  A.units = units;
-  A.split = o->ws_split_threshold ? (uint64_t)(o->ws_split_threshold + 63) / 64 * 64 : kLftjSplit;
   A.cap = kLftjTaskSlots;
   AMJ_TRY(scratch(ctx, SLOT_DYN_CTL, sizeof(WsCtl), &ctl));
   AMJ_TRY(scratch(ctx, SLOT_DYN_TASKS, A.cap * lftj_ws_task_bytes(), &tasks));
@@ -346,6 +349,17 @@ static int run_lftj_ws(amj_ctx_t* ctx, const LPlan& P_in, const amj_opts_t* o,
   // per unit
   const uint64_t fit = (uint64_t)lftj_ws_blocks_per_cu(P, final_mode) *
                        (uint64_t)ctx->props.multiProcessorCount;
+  P.rpu = kWave;
+  A.split = kLftjSplit;
+  if (o->ws_split_threshold) {
+    A.split = (uint64_t)(o->ws_split_threshold + 63) / 64 * 64;
+  } else if (lftj_static_shape(P)) {
+    while (P.rpu > 4 && P.roots / P.rpu < fit * kWavesPerBlock * kWsUnitsPerWave) P.rpu >>= 1;
+    if (P.n_attrs == 3) A.split = std::max<uint64_t>(kLftjSplit, (uint64_t)P.rpu * 64);
+    if (!A.max_claim) A.max_claim = 1;
+  }
+  const uint64_t units = lftj_units(P);
+  A.units = units;
   const unsigned grid = (unsigned)std::max<uint64_t>(
       1, std::min<uint64_t>((units + kWavesPerBlock - 1) / kWavesPerBlock, fit));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[2], s));
@@ -648,6 +662,7 @@ int alftj_trie_offload(amj_ctx_t* ctx, amj_trie_t* t) {
   if (n1) AMJ_HIP_TRY(ctx, hipMemcpyAsync(d1, t->dev.d1, n1 * 4, hipMemcpyDeviceToHost, s));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
   const uint32_t max_run = t->dev.max_run;
+  const bool distinct = t->dev.distinct;
   const double ms = t->dev.build_ms;
   free_trie(ctx, &t->dev);
   t->host = true;
@@ -657,6 +672,7 @@ int alftj_trie_offload(amj_ctx_t* ctx, amj_trie_t* t) {
   t->dev.n0 = (uint32_t)n0;
   t->dev.n1 = (uint32_t)n1;
   t->dev.max_run = max_run;
+  t->dev.distinct = distinct;
   t->dev.build_ms = ms;
   t->dev.view = LRel{d0, off, d1, nullptr, (uint32_t)n0, 0};
   return AMJ_OK;

@@ -88,7 +88,7 @@ int run_lftj_ooc(amj_ctx_t* ctx, const LPlan& P, const HostView* hv, const amj_o
       cap1 = std::max<uint64_t>(cap1, hv[r].off[hi] - hv[r].off[lo]);
     }
   }
-  const uint64_t per_rel = (cap0 * 2 + 1 + cap1) * 4 + 256;
+  const uint64_t per_rel = (cap0 * 2 + 1 + cap1 + kTriePad) * 4 + 256;
   void* buf[2] = {nullptr, nullptr};
   AMJ_TRY(scratch(ctx, SLOT_OOC_A, per_rel * R, &buf[0]));
   AMJ_TRY(scratch(ctx, SLOT_OOC_B, per_rel * R, &buf[1]));

@@ -149,6 +149,7 @@ int build_trie(amj_ctx_t* ctx, const int32_t* c0, const int32_t* c1, uint64_t n,
     return AMJ_ERR_ARG;
   }
   hipStream_t s = ctx->stream;
+  out->distinct = true;  // duplicate pairs are dropped
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[0], s));
   if (n == 0) {
     AMJ_TRY(dmalloc(ctx, (void**)&out->off, 4));
@@ -175,7 +176,7 @@ int build_trie(amj_ctx_t* ctx, const int32_t* c0, const int32_t* c1, uint64_t n,
   uint32_t m = 0;
   AMJ_HIP_TRY(ctx, hipMemcpyAsync(&m, (uint32_t*)pos + n, 4, hipMemcpyDeviceToHost, s));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
-  AMJ_TRY(dmalloc(ctx, (void**)&out->d1, (uint64_t)m * 4));
+  AMJ_TRY(dmalloc(ctx, (void**)&out->d1, ((uint64_t)m + kTriePad) * 4));
   out->n1 = m;
   hipLaunchKernelGGL(trie_compact_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s,
                      (const uint64_t*)keys, n, (const uint32_t*)pos, (const uint32_t*)keep,
@@ -210,6 +211,7 @@ int trie_from_host(amj_ctx_t* ctx, uint64_t n0, const int32_t* d0, const uint64_
     return AMJ_ERR_ARG;
   }
   std::vector<uint32_t> off32(n0 + 1);
+  out->distinct = true;
   for (uint64_t j = 0; j < n0; ++j) {
     if (off[j + 1] < off[j] || (j > 0 && d0[j] <= d0[j - 1])) {
       set_error(ctx, AMJ_ERR_ARG, "trie level 0 must be strictly increasing with monotone offsets");
@@ -219,6 +221,8 @@ int trie_from_host(amj_ctx_t* ctx, uint64_t n0, const int32_t* d0, const uint64_
       if (d1[k] < d1[k - 1]) {
         set_error(ctx, AMJ_ERR_ARG, "trie child lists must be sorted");
         return AMJ_ERR_ARG;
+      } else if (d1[k] == d1[k - 1]) {
+        out->distinct = false;
       }
     off32[j] = (uint32_t)off[j];
   }
@@ -228,7 +232,7 @@ int trie_from_host(amj_ctx_t* ctx, uint64_t n0, const int32_t* d0, const uint64_
   AMJ_TRY(dmalloc(ctx, (void**)&out->d0, n0 * 4));
   out->n0 = (uint32_t)n0;
   AMJ_TRY(dmalloc(ctx, (void**)&out->off, (n0 + 1) * 4));
-  AMJ_TRY(dmalloc(ctx, (void**)&out->d1, n1 * 4));
+  AMJ_TRY(dmalloc(ctx, (void**)&out->d1, (n1 + kTriePad) * 4));
   out->n1 = (uint32_t)n1;
   if (n0) AMJ_HIP_TRY(ctx, hipMemcpyAsync(out->d0, d0, n0 * 4, hipMemcpyHostToDevice, s));
   if (n1) AMJ_HIP_TRY(ctx, hipMemcpyAsync(out->d1, d1, n1 * 4, hipMemcpyHostToDevice, s));
@@ -242,7 +246,7 @@ void free_trie(amj_ctx_t* ctx, TrieDev* t) {
   if (ctx) (void)hipStreamSynchronize(ctx->stream);
   dfree(ctx, t->d0, (uint64_t)t->n0 * 4);
   dfree(ctx, t->off, ((uint64_t)t->n0 + 1) * 4);
-  dfree(ctx, t->d1, (uint64_t)t->n1 * 4);
+  dfree(ctx, t->d1, ((uint64_t)t->n1 + kTriePad) * 4);
   dfree(ctx, t->vrange, (uint64_t)t->vrange_n * 8);
   *t = TrieDev{};
 }

@@ -192,8 +192,14 @@ __host__ __device__ __forceinline__ uint32_t rotl32(uint32_t x, uint32_t r) {
 size_t scan_temp_elems(uint64_t n);
 hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* temp,
                               hipStream_t s);
+// last (device-visible, may be nullptr) also receives the last output element.
 hipError_t exclusive_scan_u64(const uint64_t* in, uint64_t* out, uint64_t n, uint64_t* temp,
-                              hipStream_t s);
+                              hipStream_t s, uint64_t* last = nullptr);
+// out[0], out[1] (device-visible) = the sums of a[0 .. n) and b[0 .. n) (b == nullptr: 0); temp
+// holds kSumPairTemp words.
+constexpr uint64_t kSumPairTemp = 512;
+hipError_t sum_pair_u64(const uint64_t* a, const uint64_t* b, uint64_t n, uint64_t* out,
+                        uint64_t* temp, hipStream_t s);
 // Sum of n u64 values into *out (device pointer).
 hipError_t reduce_sum_u64(const uint64_t* in, uint64_t n, uint64_t* out, uint64_t* temp,
                           hipStream_t s);
@@ -267,7 +273,7 @@ hipError_t launch_chunk_fill(const ProbeOut& out, int n_attrs, const uint64_t* t
                              const uint64_t* tpre, uint64_t n_chunks, uint32_t chunk, uint64_t n,
                              uint64_t reserved, hipStream_t s);
 
-// Count pass: per-unit result counts (unit = 64 consecutive probe rows).
+// Count pass: per-unit result counts (unit = 64 consecutive probe rows); counts[units] = 0.
 hipError_t launch_probe_count(const Plan& plan, uint64_t* unit_counts, hipStream_t s);
 // Write pass: units write at unit_base[u] (exclusive scan of counts); per-block checksum
 // partials go to block_sums. hash=false skips the checksum when materialising.

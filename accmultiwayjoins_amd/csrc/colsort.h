@@ -109,4 +109,7 @@ struct ColSortFacts {
 hipError_t run_col_sort(const ColSort& c, void* temp, uint64_t* mail, hipEvent_t known,
                         hipStream_t s, ColSortFacts* facts);
 
+// The same for at most kHashSmallRows rows (hashbuild.hip): one launch, no buffers, no wait.
+hipError_t launch_small_sort(const ColSort& c, hipStream_t s);
+
 }  // namespace amj

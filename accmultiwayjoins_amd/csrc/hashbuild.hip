@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kSmallThreads) void hash_small_kernel(
   uint64_t key[ITEMS];
   uint64_t diff = 0;
   bool out = false;
-  with_rows(c, nullptr, [&](auto load) {
+  with_rows(c, c.in64, [&](auto load) {
     const uint64_t k0 = load(0);
 #pragma unroll
     for (int r = 0; r < ITEMS; ++r) {
@@ -219,6 +219,7 @@ __global__ __launch_bounds__(kSmallThreads) void hash_small_kernel(
     const uint32_t i = base + (uint32_t)r * kWave;
     if (i < n) col_store(c, i, key[r]);
   }
+  if (!ptrs) return;
   const uint32_t buckets = 1u << log_b;
   const auto bucket = [&](uint32_t i) {
     return log_b == 0 ? 0u : (uint32_t)(tile[i] >> 32) >> (32u - log_b);
@@ -260,6 +261,10 @@ hipError_t launch_hash_small(const ColSort& c, uint32_t log_b, uint32_t* ptrs, u
   else LAUNCH(8);
 #undef LAUNCH
   return hipGetLastError();
+}
+
+hipError_t launch_small_sort(const ColSort& c, hipStream_t s) {
+  return launch_hash_small(c, 0, nullptr, nullptr, nullptr, s);
 }
 
 // Bucket bounds of sorted composites (the pairwise engine's partitions).

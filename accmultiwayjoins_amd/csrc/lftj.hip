@@ -69,6 +69,7 @@ __global__ __launch_bounds__(kBlock) void lftj_count_kernel(const LPlan P,
                                                             uint64_t units,
                                                             const uint64_t* __restrict__ order) {
   const uint64_t k = (uint64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+  if (blockIdx.x == 0 && threadIdx.x == 0) counts[units] = 0;  // the scan leaves the total there
   if (k >= units) return;  // no barriers in this kernel
   const uint64_t unit = unit_of(order, k);
   LLv<A> l0;

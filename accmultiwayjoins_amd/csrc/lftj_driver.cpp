@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "colsort.h"
 #include "lftj.h"
 #include "probe_common.h"
 #include "runtime.h"
@@ -116,14 +117,26 @@ static int unit_order(amj_ctx_t* ctx, const LPlan& P, const uint64_t** order) {
   const uint64_t units = lftj_units(P);
   if (units < kLftjOrderMinUnits) return AMJ_OK;
   hipStream_t s = ctx->stream;
-  void *keys = nullptr, *alt = nullptr, *tmp = nullptr;
+  void *keys = nullptr, *alt = nullptr, *out = nullptr, *tmp = nullptr;
   AMJ_TRY(scratch(ctx, SLOT_SORT_KEYS, units * 8, &keys));
   AMJ_TRY(scratch(ctx, SLOT_SORT_ALT, units * 8, &alt));
-  AMJ_TRY(scratch(ctx, SLOT_SORT_TEMP, radix_sort_temp_bytes(units), &tmp));
+  AMJ_TRY(scratch(ctx, SLOT_LFTJ_ORDER, units * 8, &out));
   AMJ_HIP_TRY(ctx, launch_lftj_unit_weights(P, (uint64_t*)keys, s));
-  // the weight bytes only: the sort is stable, so equal weights keep unit order
-  AMJ_HIP_TRY(ctx, radix_sort_u64((uint64_t*)keys, (uint64_t*)alt, units, 0xf0u, tmp, s));
-  *order = (const uint64_t*)keys;
+  // the upper two bytes of the weight (sign, exponent, seven bits of mantissa) are order enough
+  ColSort c;
+  c.in64 = (const uint64_t*)keys;
+  c.n = units;
+  c.mask = 0xc0u;
+  c.buf_x = (uint64_t*)alt;
+  c.buf_y = c.out64 = (uint64_t*)out;
+  if (units <= kHashSmallRows) {
+    AMJ_HIP_TRY(ctx, launch_small_sort(c, s));
+  } else {
+    AMJ_TRY(scratch(ctx, SLOT_SORT_TEMP, col_sort_temp_bytes(units), &tmp));
+    ColSortFacts facts;
+    AMJ_HIP_TRY(ctx, run_col_sort(c, tmp, ctx->mail + MAIL_SORT, ctx->ev[6], s, &facts));
+  }
+  *order = (const uint64_t*)out;
   return AMJ_OK;
 }
 
@@ -274,10 +287,11 @@ static int run_lftj_count(amj_ctx_t* ctx, const LPlan& P, amj_result_t* res) {
   AMJ_HIP_TRY(ctx, launch_lftj_write(P, nullptr, LOut{}, true, (uint64_t*)bsum, &nb_used, order,
                                      s, (uint64_t*)bcnt));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[4], s));
-  AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bsum, nb_used, &res->checksum));
-  AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bcnt, nb_used, &res->count));
+  AMJ_TRY(enqueue_totals(ctx, (const uint64_t*)bsum, (const uint64_t*)bcnt, nb_used));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[5], s));
   AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[5]));
+  res->checksum = mail_word(ctx, MAIL_TOTALS);
+  res->count = mail_word(ctx, MAIL_TOTALS + 1);
   res->probe_ms = elapsed_ms(ctx->ev[2], ctx->ev[5]);
   res->probe_kernel_ms = elapsed_ms(ctx->ev[3], ctx->ev[4]);
   res->probe_kernel_launches = 1;
@@ -472,13 +486,12 @@ static int run_lftj_dfs(amj_ctx_t* ctx, const LPlan& P, const amj_opts_t* o, amj
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[2], s));
   const uint64_t* order = nullptr;
   AMJ_TRY(unit_order(ctx, P, &order));
-  AMJ_HIP_TRY(ctx, hipMemsetAsync(counts, 0, (units + 1) * 8, s));
+  if (units == 0) AMJ_HIP_TRY(ctx, hipMemsetAsync(counts, 0, 8, s));
   AMJ_HIP_TRY(ctx, launch_lftj_count(P, (uint64_t*)counts, order, s));
   AMJ_HIP_TRY(ctx, exclusive_scan_u64((uint64_t*)counts, (uint64_t*)counts, units + 1,
-                                      (uint64_t*)tmp, s));
-  uint64_t total = 0;
-  AMJ_HIP_TRY(ctx, hipMemcpyAsync(&total, (uint64_t*)counts + units, 8, hipMemcpyDeviceToHost, s));
+                                      (uint64_t*)tmp, s, ctx->mail + MAIL_COUNT));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
+  const uint64_t total = mail_word(ctx, MAIL_COUNT);
   res->count = total;
   LOut out{};
   if (o->materialize && total > 0) {
@@ -500,9 +513,10 @@ static int run_lftj_dfs(amj_ctx_t* ctx, const LPlan& P, const amj_opts_t* o, amj
   AMJ_HIP_TRY(ctx, launch_lftj_write(P, (const uint64_t*)counts, out, hash, (uint64_t*)bsum,
                                      &nb_used, order, s));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[4], s));
-  if (hash) AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bsum, nb_used, &res->checksum));
+  if (hash) AMJ_TRY(enqueue_totals(ctx, (const uint64_t*)bsum, nullptr, nb_used));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[5], s));
   AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[5]));
+  if (hash) res->checksum = mail_word(ctx, MAIL_TOTALS);
   res->probe_ms = elapsed_ms(ctx->ev[2], ctx->ev[5]);
   res->probe_kernel_ms = elapsed_ms(ctx->ev[3], ctx->ev[4]);
   res->probe_kernel_launches = 1;

@@ -32,6 +32,7 @@ __global__ __launch_bounds__(kBlock) void probe_count_kernel(const Plan P,
                                                              uint64_t* __restrict__ counts,
                                                              uint64_t units) {
   const uint64_t unit = (uint64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+  if (blockIdx.x == 0 && threadIdx.x == 0) counts[units] = 0;  // the scan leaves the total there
   if (unit >= units) return;  // whole wave leaves; this kernel has no barriers
   LvL<L> l0;
   make_level0(P, unit * kWave, l0);

@@ -460,14 +460,18 @@ int alloc_output(amj_ctx_t* ctx, uint64_t rows, int n_attrs, amj_result_t* res) 
   return AMJ_OK;
 }
 
-int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb,
-                           uint64_t* out) {
-  void *sum = nullptr, *tmp = nullptr;
-  AMJ_TRY(scratch(ctx, SLOT_SUM, 64, &sum));
-  AMJ_TRY(scratch(ctx, SLOT_SCAN_TEMP, scan_temp_elems(nb) * 8, &tmp));
-  AMJ_HIP_TRY(ctx, reduce_sum_u64(block_sums, nb, (uint64_t*)sum, (uint64_t*)tmp, ctx->stream));
-  AMJ_HIP_TRY(ctx, hipMemcpyAsync(out, sum, 8, hipMemcpyDeviceToHost, ctx->stream));
+int enqueue_totals(amj_ctx_t* ctx, const uint64_t* sums, const uint64_t* counts, uint64_t nb) {
+  void* tmp = nullptr;
+  AMJ_TRY(scratch(ctx, SLOT_SUM, (kSumPairTemp + 8) * 8, &tmp));
+  AMJ_HIP_TRY(ctx, sum_pair_u64(sums, counts, nb, ctx->mail + MAIL_TOTALS, (uint64_t*)tmp + 8,
+                                ctx->stream));
+  return AMJ_OK;
+}
+
+int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb, uint64_t* out) {
+  AMJ_TRY(enqueue_totals(ctx, block_sums, nullptr, nb));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  *out = mail_word(ctx, MAIL_TOTALS);
   return AMJ_OK;
 }
 
@@ -498,10 +502,11 @@ static int run_plain_count(amj_ctx_t* ctx, Plan& P, amj_result_t* res) {
   AMJ_HIP_TRY(ctx, launch_probe_write(P, nullptr, ProbeOut{}, true, (uint64_t*)bsum, &nb_used, s,
                                       (uint64_t*)bcnt));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[4], s));
-  AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bsum, nb_used, &res->checksum));
-  AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bcnt, nb_used, &res->count));
+  AMJ_TRY(enqueue_totals(ctx, (const uint64_t*)bsum, (const uint64_t*)bcnt, nb_used));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[5], s));
   AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[5]));
+  res->checksum = mail_word(ctx, MAIL_TOTALS);
+  res->count = mail_word(ctx, MAIL_TOTALS + 1);
   res->probe_ms = elapsed_ms(ctx->ev[2], ctx->ev[5]);
   res->probe_kernel_ms = elapsed_ms(ctx->ev[3], ctx->ev[4]);
   res->probe_kernel_launches = 1;
@@ -519,13 +524,12 @@ static int run_plain(amj_ctx_t* ctx, Plan& P, const amj_opts_t* o, amj_result_t*
   AMJ_TRY(scratch(ctx, SLOT_UNIT_COUNTS, (units + 1) * 8, &counts));
   AMJ_TRY(scratch(ctx, SLOT_SCAN_TEMP, scan_temp_elems(units + 1) * 8, &tmp));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[2], s));
-  AMJ_HIP_TRY(ctx, hipMemsetAsync(counts, 0, (units + 1) * 8, s));
+  if (units == 0) AMJ_HIP_TRY(ctx, hipMemsetAsync(counts, 0, 8, s));
   AMJ_HIP_TRY(ctx, launch_probe_count(P, (uint64_t*)counts, s));
   AMJ_HIP_TRY(ctx, exclusive_scan_u64((uint64_t*)counts, (uint64_t*)counts, units + 1,
-                                      (uint64_t*)tmp, s));
-  uint64_t total = 0;
-  AMJ_HIP_TRY(ctx, hipMemcpyAsync(&total, (uint64_t*)counts + units, 8, hipMemcpyDeviceToHost, s));
+                                      (uint64_t*)tmp, s, ctx->mail + MAIL_COUNT));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
+  const uint64_t total = mail_word(ctx, MAIL_COUNT);
   res->count = total;
 
   ProbeOut out{};
@@ -549,9 +553,10 @@ static int run_plain(amj_ctx_t* ctx, Plan& P, const amj_opts_t* o, amj_result_t*
   AMJ_HIP_TRY(ctx, launch_probe_write(P, (const uint64_t*)counts, out, hash, (uint64_t*)bsum,
                                       &nb_used, s));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[4], s));
-  if (hash) AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bsum, nb_used, &res->checksum));
+  if (hash) AMJ_TRY(enqueue_totals(ctx, (const uint64_t*)bsum, nullptr, nb_used));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[5], s));
   AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[5]));
+  if (hash) res->checksum = mail_word(ctx, MAIL_TOTALS);
   res->probe_ms = elapsed_ms(ctx->ev[2], ctx->ev[5]);
   res->probe_kernel_ms = elapsed_ms(ctx->ev[3], ctx->ev[4]);
   res->probe_kernel_launches = 1;

@@ -90,14 +90,12 @@ enum ScratchSlot {
   SLOT_MISC2,
   SLOT_MISC3,
   SLOT_TRIE0,
-  SLOT_TRIE1,
-  SLOT_TRIE2,
-  SLOT_TRIE3,
   SLOT_PROBE_SORTED,  // frequent-item path: probe columns grouped by join key
   SLOT_DYN_CTL,    // persistent probe: control block, task records, task flags
   SLOT_DYN_TASKS,
   SLOT_DYN_READY,
   SLOT_TUNE_SAMPLE,  // the autotuner's probe samples (the engines it runs use the others)
+  SLOT_LFTJ_ORDER,   // the triejoin's launch order of units
   SLOT_LFTJ_SAMPLE,  // the triejoin's output-size sample: window offsets of the sampled roots
 };
 
@@ -118,7 +116,15 @@ uint64_t arena_largest(const amj_ctx_t* ctx);
 int scratch(amj_ctx_t* ctx, int slot, size_t bytes, void** out);
 
 // Words of amj_ctx::mail.
-enum MailWord { MAIL_KEY_RANGE = 0, MAIL_SORT = 2, MAIL_WORDS = 64 };
+enum MailWord {
+  MAIL_KEY_RANGE = 0,
+  MAIL_SORT = 2,       // 2 words
+  MAIL_TOTALS = 4,     // 2 words: enqueue_totals
+  MAIL_COUNT = 6,      // result rows of a count pass
+  MAIL_TRIE = 8,       // 4 words
+  MAIL_FIB = 16,       // kMaxLevels + 1 words
+  MAIL_WORDS = 64
+};
 
 // Bytes that hbm_budget_bytes counts as held: the bucket records, which only speed lookups up and
 // are not built when memory is short, are not among them.
@@ -158,6 +164,12 @@ double elapsed_ms(hipEvent_t a, hipEvent_t b);
 bool fib_eligible(const Plan& P);
 int alloc_output(amj_ctx_t* ctx, uint64_t rows, int n_attrs, amj_result_t* res);
 int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb, uint64_t* out);
+// Enqueue the sums of nb per-block checksums and (may be nullptr) counts; they are read with
+// mail_word(ctx, MAIL_TOTALS) and + 1 once the stream has been waited for.
+int enqueue_totals(amj_ctx_t* ctx, const uint64_t* sums, const uint64_t* counts, uint64_t nb);
+inline uint64_t mail_word(const amj_ctx_t* ctx, int word) {
+  return ((const volatile uint64_t*)ctx->mail)[word];
+}
 uint64_t budget_left(amj_ctx_t* ctx, const amj_opts_t* o);
 // Frequent-item path: suffix tables + output-window writer. AMJ_ERR_STATE asks the caller to
 // use the count/write path instead (a frontier level would exceed 2^32 children).

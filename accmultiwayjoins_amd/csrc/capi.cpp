@@ -102,7 +102,8 @@ int amj_ctx_create(int device, amj_ctx_t** out) {
   for (auto& e : ctx->ev)
     if (hipEventCreate(&e) != hipSuccess) return AMJ_ERR_HIP;
   if (hipHostMalloc((void**)&ctx->mail, MAIL_WORDS * sizeof(uint64_t), hipHostMallocDefault) !=
-      hipSuccess)
+      hipSuccess ||
+      hipHostMalloc((void**)&ctx->staging, kStaging, hipHostMallocDefault) != hipSuccess)
     return AMJ_ERR_HIP;
   *out = ctx.release();
   return AMJ_OK;
@@ -112,12 +113,15 @@ void amj_ctx_destroy(amj_ctx_t* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   (void)hipDeviceSynchronize();
+  ctx->closing = true;
+  park_clear(ctx);
   for (auto& kv : ctx->scratch) dfree(ctx, kv.second.p, kv.second.bytes);
   pool_clear(ctx);
   if (ctx->arena.base) dfree(ctx, ctx->arena.base, ctx->arena.size);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
   if (ctx->mail) (void)hipHostFree(ctx->mail);
+  if (ctx->staging) (void)hipHostFree(ctx->staging);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   delete ctx;
@@ -165,6 +169,11 @@ int amj_device_info(amj_ctx_t* ctx, char* name, size_t name_len, uint64_t* hbm_b
   return AMJ_OK;
 }
 
+// Device bytes of one column of a relation that the library holds.
+static size_t owned_col_bytes(uint64_t rows) {
+  return (std::max<uint64_t>(rows, 1) * 4 + 255) / 256 * 256;
+}
+
 int amj_relation_create(amj_ctx_t* ctx, const amj_rel_t* r, amj_relation_t** out) {
   if (!ctx || !r || !out) return AMJ_ERR_ARG;
   *out = nullptr;
@@ -186,17 +195,42 @@ int amj_relation_create(amj_ctx_t* ctx, const amj_rel_t* r, amj_relation_t** out
   }
   for (uint32_t c = 0; c < r->num_cols; ++c) {
     rel->attr_ids[c] = r->attr_ids ? r->attr_ids[c] : c;
-    if (r->on_device) {
-      rel->cols[c] = const_cast<int32_t*>(r->cols[c]);
-    } else {
-      AMJ_TRY(dmalloc(ctx, (void**)&rel->cols[c], std::max<uint64_t>(r->rows, 1) * 4));
-      if (r->rows)
-        AMJ_HIP_TRY(ctx, hipMemcpyAsync(rel->cols[c], r->cols[c], r->rows * 4,
-                                        hipMemcpyHostToDevice, ctx->stream));
-    }
+    if (r->on_device) rel->cols[c] = const_cast<int32_t*>(r->cols[c]);
   }
   rel->owned = !r->on_device;
-  AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  if (rel->owned) {
+    // one block for all columns, each 256-byte aligned
+    const size_t bytes = r->rows * 4, step = owned_col_bytes(r->rows);
+    AMJ_TRY(dmalloc(ctx, (void**)&rel->cols[0], step * r->num_cols));
+    for (uint32_t c = 1; c < r->num_cols; ++c)
+      rel->cols[c] = (int32_t*)((char*)rel->cols[0] + step * c);
+    int rc = AMJ_OK;
+    if (bytes > 0 && step * r->num_cols <= kStagedCopy) {
+      const void* src[AMJ_MAX_PROBE_COLS];
+      size_t at[AMJ_MAX_PROBE_COLS], n[AMJ_MAX_PROBE_COLS];
+      for (uint32_t c = 0; c < r->num_cols; ++c) {
+        src[c] = r->cols[c];
+        at[c] = step * c;
+        n[c] = bytes;
+      }
+      rc = stage_upload(ctx, rel->cols[0], src, at, n, (int)r->num_cols);
+    } else if (bytes > 0) {
+      hipError_t e = hipSuccess;
+      for (uint32_t c = 0; c < r->num_cols && e == hipSuccess; ++c)
+        e = hipMemcpyAsync(rel->cols[c], r->cols[c], bytes, hipMemcpyHostToDevice, ctx->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+      if (e != hipSuccess) {
+        set_error(ctx, AMJ_ERR_HIP, std::string("relation upload: ") + hipGetErrorString(e));
+        rc = AMJ_ERR_HIP;
+      }
+    }
+    if (rc != AMJ_OK) {
+      dfree(ctx, rel->cols[0], step * r->num_cols);
+      return rc;
+    }
+  } else {
+    AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  }
   *out = rel.release();
   return AMJ_OK;
 }
@@ -205,8 +239,7 @@ void amj_relation_destroy(amj_ctx_t* ctx, amj_relation_t* rel) {
   if (!rel) return;
   if (rel->owned) {
     if (ctx) (void)hipStreamSynchronize(ctx->stream);
-    for (uint32_t c = 0; c < rel->num_cols; ++c)
-      dfree(ctx, rel->cols[c], std::max<uint64_t>(rel->rows, 1) * 4);
+    dfree(ctx, rel->cols[0], owned_col_bytes(rel->rows) * rel->num_cols);
   }
   delete rel;
 }
@@ -349,6 +382,7 @@ int amj_result_copy_col(amj_ctx_t* ctx, const amj_result_t* res, uint32_t col, u
     return AMJ_ERR_ARG;
   }
   if (n == 0) return AMJ_OK;
+  if (n * 4 <= kStagedCopy) return stage_download(ctx, host_out, res->cols[col] + row0, n * 4);
   AMJ_HIP_TRY(ctx, hipMemcpyAsync(host_out, res->cols[col] + row0, n * 4, hipMemcpyDeviceToHost,
                                   ctx->stream));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));

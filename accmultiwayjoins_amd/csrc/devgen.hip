@@ -228,7 +228,9 @@ int amj_device_alloc(amj_ctx_t* ctx, size_t bytes, void** out) {
 }
 
 void amj_device_free(amj_ctx_t* ctx, void* p, size_t bytes) {
-  if (ctx && p) dfree(ctx, p, bytes ? bytes : 1);
+  if (!ctx || !p) return;
+  (void)hipDeviceSynchronize();  // the caller's work on it may be on streams of its own
+  dfree(ctx, p, bytes ? bytes : 1);
 }
 
 int amj_memcpy(amj_ctx_t* ctx, void* dst, const void* src, size_t bytes) {

@@ -26,31 +26,99 @@ double elapsed_ms(hipEvent_t a, hipEvent_t b) {
   return (double)ms;
 }
 
+// Bytes allocated for a request: classes an eighth of a power of two apart, so that sizes that
+// differ a little share parked blocks.
+static size_t block_bytes(size_t bytes) {
+  if (bytes == 0) bytes = 256;
+  if (bytes > kParkBlock) return bytes;
+  size_t g = 256;
+  while (g * 16 < bytes) g <<= 1;
+  return (bytes + g - 1) / g * g;
+}
+
+void park_clear(amj_ctx_t* ctx) {
+  for (auto& b : ctx->parked) (void)hipFree(b.p);
+  ctx->parked.clear();
+  ctx->parked_bytes = 0;
+}
+
 int dmalloc(amj_ctx_t* ctx, void** p, size_t bytes) {
   *p = nullptr;
-  if (bytes == 0) bytes = 256;
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && !ctx->out_pool.empty()) {  // parked result buffers give way first
-    (void)hipGetLastError();
-    pool_clear(ctx);
-    e = hipMalloc(p, bytes);
+  const size_t size = block_bytes(bytes);
+  for (size_t i = ctx->parked.size(); i-- > 0;)
+    if (ctx->parked[i].bytes == size) {
+      *p = ctx->parked[i].p;
+      ctx->parked.erase(ctx->parked.begin() + (std::ptrdiff_t)i);
+      ctx->parked_bytes -= size;
+      break;
+    }
+  if (!*p) {
+    hipError_t e = hipMalloc(p, size);
+    if (e != hipSuccess && !(ctx->out_pool.empty() && ctx->parked.empty())) {
+      (void)hipGetLastError();  // parked blocks and result buffers give way first
+      pool_clear(ctx);
+      park_clear(ctx);
+      e = hipMalloc(p, size);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      *p = nullptr;
+      set_error(ctx, AMJ_ERR_NOMEM,
+                "hipMalloc(" + std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
+      return AMJ_ERR_NOMEM;
+    }
   }
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    set_error(ctx, AMJ_ERR_NOMEM,
-              "hipMalloc(" + std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
-    return AMJ_ERR_NOMEM;
-  }
-  ctx->allocated += bytes;
+  ctx->allocated += bytes ? bytes : 256;
   ctx->peak = std::max(ctx->peak, ctx->allocated);
   return AMJ_OK;
 }
 
-void dfree(amj_ctx_t* ctx, void* p, size_t bytes) {
+static void release_block(amj_ctx_t* ctx, void* p, size_t bytes, bool park) {
   if (!p) return;
-  (void)hipFree(p);
-  if (bytes == 0) bytes = 256;
-  if (ctx) ctx->allocated -= std::min<uint64_t>(ctx->allocated, bytes);
+  const size_t size = block_bytes(bytes);
+  if (ctx) ctx->allocated -= std::min<uint64_t>(ctx->allocated, bytes ? bytes : 256);
+  if (!ctx || !park || ctx->closing || size > kParkBlock) {
+    (void)hipFree(p);
+    return;
+  }
+  ctx->parked.push_back(amj_ctx::Buf{p, size});
+  ctx->parked_bytes += size;
+  while (ctx->parked_bytes > kParkTotal || ctx->parked.size() > kParkCount) {
+    const amj_ctx::Buf b = ctx->parked.front();
+    ctx->parked.erase(ctx->parked.begin());
+    ctx->parked_bytes -= b.bytes;
+    (void)hipFree(b.p);
+  }
+}
+
+void dfree(amj_ctx_t* ctx, void* p, size_t bytes) { release_block(ctx, p, bytes, true); }
+
+int stage_upload(amj_ctx_t* ctx, void* dst, const void* const* src, const size_t* at,
+                 const size_t* bytes, int n) {
+  const size_t total = (at[n - 1] + bytes[n - 1] + 255) / 256 * 256;
+  if (ctx->staging_used + total > kStaging) {  // earlier copies may still be reading it
+    AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->staging_used = 0;
+  }
+  char* p = ctx->staging + ctx->staging_used;
+  for (int i = 0; i < n; ++i) std::memcpy(p + at[i], src[i], bytes[i]);
+  AMJ_HIP_TRY(ctx, hipMemcpyAsync(dst, p, at[n - 1] + bytes[n - 1], hipMemcpyHostToDevice,
+                                  ctx->stream));
+  ctx->staging_used += total;
+  return AMJ_OK;
+}
+
+int stage_download(amj_ctx_t* ctx, void* dst, const void* src, size_t bytes) {
+  if (ctx->staging_used + bytes > kStaging) {
+    AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->staging_used = 0;
+  }
+  char* p = ctx->staging + ctx->staging_used;
+  AMJ_HIP_TRY(ctx, hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+  AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->staging_used = 0;
+  std::memcpy(dst, p, bytes);
+  return AMJ_OK;
 }
 
 int scratch(amj_ctx_t* ctx, int slot, size_t bytes, void** out) {
@@ -327,12 +395,12 @@ void pool_put(amj_ctx_t* ctx, void* p, size_t bytes) {
     const amj_ctx::Buf b = ctx->out_pool.front();
     ctx->out_pool.erase(ctx->out_pool.begin());
     ctx->pool_bytes -= b.bytes;
-    dfree(ctx, b.p, b.bytes);
+    release_block(ctx, b.p, b.bytes, false);
   }
 }
 
 void pool_clear(amj_ctx_t* ctx) {
-  for (auto& b : ctx->out_pool) dfree(ctx, b.p, b.bytes);
+  for (auto& b : ctx->out_pool) release_block(ctx, b.p, b.bytes, false);
   ctx->out_pool.clear();
   ctx->pool_bytes = 0;
 }
@@ -478,7 +546,7 @@ int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb, uin
 uint64_t budget_left(amj_ctx_t* ctx, const amj_opts_t* o) {
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-  uint64_t left = free_b + ctx->pool_bytes;  // parked buffers are reusable
+  uint64_t left = free_b + ctx->pool_bytes + ctx->parked_bytes;  // given back when needed
   if (ctx->arena.base) left = arena_largest(ctx);
   if (o && o->hbm_budget_bytes) {
     const uint64_t held = budget_held(ctx);

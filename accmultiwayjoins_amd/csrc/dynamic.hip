@@ -134,8 +134,8 @@ __global__ __launch_bounds__(kBlock) void dyn_kernel(const Plan P, const ProbeOu
   Acc acc{};
   ws_serve(
       A,
-      [&](uint64_t u, uint64_t ue) {
-        for (uint64_t v = u; v < ue; ++v) {
+      [&](uint64_t u, uint64_t ue, uint64_t step) {
+        for (uint64_t v = u; v < ue; v += step) {
           LvL<L> l0;
           make_level0(P, v * kWave, l0);
           if (l0.T) dyn_descend<L, 0, MODE>(P, l0, 0, l0.T, out, A, acc, W);
@@ -270,7 +270,7 @@ int run_dynamic(amj_ctx_t* ctx, Plan& P, const amj_opts_t* o, amj_result_t* res)
   const uint64_t units = probe_units(P);
   DynArgs A{};
   void *ctl = nullptr, *tasks = nullptr, *ready = nullptr;
-  AMJ_TRY(scratch(ctx, SLOT_DYN_CTL, 256, &ctl));
+  AMJ_TRY(scratch(ctx, SLOT_DYN_CTL, sizeof(DynCtl), &ctl));
   A.ctl = (DynCtl*)ctl;
   A.units = units;
   int clock_khz = 0;
@@ -442,7 +442,7 @@ static int ooc_stream(amj_ctx_t* ctx, const Plan& P, const ProbeOut& out, bool h
     AMJ_HIP_TRY(ctx, hipEventRecord(ev.copied[b], side));
     AMJ_HIP_TRY(ctx, hipStreamWaitEvent(s, ev.copied[b], 0));
     // fresh unit and task counters for the slice; count, checksum and reservations carry on
-    AMJ_HIP_TRY(ctx, hipMemsetAsync(A.ctl, 0, 3 * sizeof(unsigned long long), s));
+    AMJ_HIP_TRY(ctx, hipMemsetAsync(A.ctl, 0, offsetof(DynCtl, out_rows), s));
     if (A.split) AMJ_HIP_TRY(ctx, hipMemsetAsync(A.ready, 0, A.cap * 4, s));
     Plan Q = P;
     Q.probe_on_host = 0;
@@ -469,7 +469,7 @@ int run_ooc(amj_ctx_t* ctx, Plan& P, const amj_opts_t* o, amj_result_t* res) {
   const int nc = P.probe_ncols;
   DynArgs A{};
   void *ctl = nullptr, *tasks = nullptr, *ready = nullptr;
-  AMJ_TRY(scratch(ctx, SLOT_DYN_CTL, 256, &ctl));
+  AMJ_TRY(scratch(ctx, SLOT_DYN_CTL, sizeof(DynCtl), &ctl));
   A.ctl = (DynCtl*)ctl;
   int clock_khz = 0;
   if (hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, ctx->device) !=

@@ -312,7 +312,7 @@ constexpr uint64_t kLftjSplit = 1024;        // ALFTJ.cuh:22 BUC_THRESHOLD
 // small units claimed one at a time, heaviest first, and only runs far longer than a unit's
 // average are shared (a 4-clique's are worth more than a triangle's). R-MAT 18 / 20 with units of
 // 64 roots claimed several at a time and every run over 1,088 shared: triangles 13.9 / 32 ms,
-// 4-cliques 60 / 186 ms; so 2.2 / 5.5 ms and 45 / 185 ms.
+// 4-cliques 60 / 186 ms; so 1.5 / 4.9 ms and 45 / 180 ms.
 constexpr uint64_t kWsUnitsPerWave = 2;
 constexpr uint64_t kLftjTaskSlots = 8192;    // task records of 5,440 bytes
 constexpr uint64_t kLftjStallMs = 20000;     // no progress for this long: give up

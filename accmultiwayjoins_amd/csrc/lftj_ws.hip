@@ -173,8 +173,8 @@ __global__ __launch_bounds__(kBlock) void lftj_ws_kernel(const LPlan P, const LO
   WsWave q{false, 0u};
   ws_serve(
       W,
-      [&](uint64_t u, uint64_t ue) {
-        for (uint64_t k = u; k < ue; ++k) {
+      [&](uint64_t u, uint64_t ue, uint64_t step) {
+        for (uint64_t k = u; k < ue; k += step) {
           LLv<A> l0;
           level0<A, SH>(P, unit_of(order, k), l0);
           if (l0.T) ws_ldescend<A, 1, SH>(P, l0, 0u, l0.T, sink, W, q, stage);

@@ -5,7 +5,7 @@
 // (common-utils/cuda/GCQueue.cuh:30-107) hands them out through CAS on tagged slots, and
 // CBarrier (MHJ-GPU/CBarrier.cuh:9-46) ends the kernel when every warp is idle; none of them
 // checks capacity. Here:
-//   * persistent waves claim units (64 probe rows / 64 roots) from a counter in guided chunks;
+//   * persistent waves claim units (64 probe rows / some roots) from counters in guided chunks;
 //   * task slots are reserved with one fetch-add on the queue tail, clamped to the capacity
 //     (requests past the end get nothing, and the wave then keeps its work);
 //   * a task record is published by its own ready flag (release store after the record), and
@@ -20,18 +20,27 @@
 
 namespace amj {
 
-// Control block of one launch (zeroed by the host).
-struct WsCtl {
-  unsigned long long next_unit;  // units claimed
+// Control block of one launch (zeroed by the host). Updates of one cache line serialise across
+// the device (tens of ns each), so what is updated often has a line of its own, and units are
+// claimed from kUnitShards counters (unit u belongs to shard u % kUnitShards; a wave starts with
+// the shard of its workgroup's XCD and goes on to the others). Count of a 1 M-row chain (15,625
+// units): 1.25 ms with one counter, 0.85 with eight.
+constexpr uint32_t kUnitShards = kXcds;
+struct alignas(128) WsShard {
+  unsigned long long next;  // units of the shard claimed
+};
+struct alignas(128) WsCtl {
+  WsShard shard[kUnitShards];
   unsigned long long q_tail;     // task slots reserved (may pass cap: clamp on read)
   unsigned long long q_head;     // task slots claimed
-  unsigned long long out_rows;   // output rows reserved (the results, plus unused chunk tails)
-  unsigned long long count;      // results
+  alignas(128) unsigned long long out_rows;  // output rows reserved (the results, plus unused
+                                             // chunk tails)
+  alignas(128) unsigned long long progress;  // tasks completed, plus heartbeats
+  unsigned int busy;             // waves holding units or a task
+  unsigned int flags;            // 1: a wait hit the time limit
+  alignas(128) unsigned long long count;  // results
   unsigned long long csum;       // checksum, sum of the waves' partials mod 2^64
   unsigned long long pushed;     // tasks published
-  unsigned long long progress;   // units and tasks completed, plus heartbeats
-  unsigned int busy;             // waves holding a unit or a task
-  unsigned int flags;            // 1: a wait hit the time limit
 };
 
 constexpr uint64_t kMaxClaim = 64;  // units claimed at once by a wave
@@ -146,62 +155,70 @@ __device__ __forceinline__ int64_t try_pop(const WsArgs& A) {
 }
 
 // The persistent loop of a wave: claim units in guided chunks and run them
-// (run_units(first, end)), then take tasks (run_task(slot)) until the launch has drained.
+// (run_units(first, end, step)), then take tasks (run_task(slot)) until the launch has drained.
+//
+// A claim is one update of one counter. A wave counts as busy from its first claim until it finds
+// no work, not per claim, and reports progress from its heartbeat (ws_step) and per task: with a
+// busy, a progress and a claim update per claim, quarter-size claims down to one unit, and all
+// three counters in one line, counting 20 M probe rows (312,500 units, fan-out 1) took 9.9 ms, of
+// which the lookups are 1.2; now 2.2.
 template <typename RunUnits, typename RunTask>
 __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
                                          RunTask&& run_task) {
   uint64_t seen = ~0ull, since = 0;  // progress counter last seen, and when it last moved
+  bool units_left = true, working = false;
+  uint32_t shard = blockIdx.x % kUnitShards;  // workgroup b runs on XCD b % 8
+  int naps = 1;
+  const auto work = [&](bool on) {  // only kept for the waits for tasks
+    if (A.split && on != working && lane_id() == 0) add_relaxed(&A.ctl->busy, on ? 1u : ~0u);
+    working = on;
+  };
   for (;;) {
-    // busy counts waves holding claimed work; it only keeps idle waves around to help (a wave
-    // that leaves early costs parallelism, never work: a pusher always serves its own tasks).
-    // Guided chunks of at most 64 units: with 64 or more units per wave, half the remaining
-    // units per wave and at least 4, so cheap units do not pay shared-counter updates of their
-    // own (every claim updates one counter, and the updates serialise: a streamed 1.5 G-row
-    // probe of 23 slices of 1 M units took 316 ms with a quarter per wave and single-unit
-    // claims at the end, 224 ms with half and at least 4, where its PCIe copies alone take
-    // about 215 ms); with fewer (the triejoin's units of 64 roots, heaviest first), a quarter
-    // and at least 1: 4 units at a time took the 4-cliques of R-MAT 20 from 290 to 860 ms.
-    uint64_t u = ~0ull, nu = 0;
-    if (lane_id() == 0) {
-      const unsigned long long seen_u = ld_rlx(&A.ctl->next_unit);
-      if (seen_u < A.units) {
-        const uint64_t waves = (uint64_t)gridDim.x * kWavesPerBlock;
-        const uint64_t most = A.max_claim ? A.max_claim : kMaxClaim;
-        const bool many = A.units >= 64 * waves;
-        const uint64_t least = (many && most >= kMinClaim) ? kMinClaim : 1;
-        uint64_t k = (A.units - seen_u) / ((many ? 2 : 4) * waves);
-        k = k < least ? least : (k > most ? most : k);
-        u = add_relaxed(&A.ctl->next_unit, (unsigned long long)k);
-        nu = k;
+    // Guided chunks of at most 64 units. With 16 or more units per wave: half the remaining ones
+    // per wave and at least 4, so that cheap units do not pay for a claim each. With fewer (the
+    // triejoin's units of many roots, heaviest first): a quarter and at least 1; 4 units at a time
+    // took the 4-cliques of R-MAT 20 from 290 to 860 ms.
+    if (units_left) {
+      uint64_t u = 0, n = 0;
+      uint32_t tried = 0;
+      for (; tried < kUnitShards; ++tried) {
+        const uint64_t size = (A.units + kUnitShards - 1 - shard) / kUnitShards;
+        if (lane_id() == 0) {
+          unsigned long long* next = &A.ctl->shard[shard].next;
+          const unsigned long long at = ld_rlx(next);
+          if (at < size) {
+            const uint64_t waves = (uint64_t)gridDim.x * kWavesPerBlock;
+            const uint64_t most = A.max_claim ? A.max_claim : kMaxClaim;
+            const bool many = A.units >= 16 * waves;
+            const uint64_t least = (many && most >= kMinClaim) ? kMinClaim : 1;
+            uint64_t k = (size - at) * kUnitShards / ((many ? 2 : 4) * waves);
+            k = k < least ? least : (k > most ? most : k);
+            u = add_relaxed(next, (unsigned long long)k);
+            n = u < size ? (k < size - u ? k : size - u) : 0;
+          }
+        }
+        n = lane0_u64(n);
+        if (n) break;
+        shard = (shard + 1) % kUnitShards;  // this one is used up, and stays so
       }
-    }
-    u = lane0_u64(u);
-    nu = lane0_u64(nu);
-    if (u < A.units) {
-      const uint64_t ue = u + nu < A.units ? u + nu : A.units;
-      // busy and progress only serve the waits for tasks: without sharing a wave leaves when
-      // the units run out, and the claim's one counter update is all it pays (the counters
-      // share a cache line, whose updates serialise: 1 M units of a 64 M-row probe slice took
-      // 16.4 ms with three updates per claim, against 6.8 ms for the same rows in one launch)
-      if (A.split && lane_id() == 0) add_relaxed(&A.ctl->busy, 1u);
-      run_units(u, ue);
-      if (A.split && lane_id() == 0) {
-        add_relaxed(&A.ctl->progress, 1ull);
-        add_relaxed(&A.ctl->busy, ~0u);
+      if (n) {
+        work(true);
+        const uint64_t first = lane0_u64(u) * kUnitShards + shard;
+        run_units(first, first + n * kUnitShards, kUnitShards);
+        continue;
       }
-      continue;
+      units_left = false;
     }
     if (A.split == 0) break;  // without sharing there are no tasks to wait for
     const int64_t slot = try_pop(A);
     if (slot >= 0) {
-      if (lane_id() == 0) add_relaxed(&A.ctl->busy, 1u);
+      work(true);
       run_task((uint64_t)slot);
-      if (lane_id() == 0) {
-        add_relaxed(&A.ctl->progress, 1ull);
-        add_relaxed(&A.ctl->busy, ~0u);
-      }
+      if (lane_id() == 0) add_relaxed(&A.ctl->progress, 1ull);
+      naps = 1;
       continue;
     }
+    work(false);
     if (slot == -2) break;
     uint32_t done = 0;
     if (lane_id() == 0)
@@ -218,7 +235,10 @@ __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
         __hip_atomic_fetch_or(&A.ctl->flags, kFlagSpin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       break;
     }
-    __builtin_amdgcn_s_sleep(64);
+    // idle waves look again after 2, 4, .. 14 us, so that thousands of them leave the counters to
+    // the waves that work
+    for (int i = 0; i < naps; ++i) __builtin_amdgcn_s_sleep(64);
+    naps = naps < 8 ? 2 * naps : 8;
   }
 }
 

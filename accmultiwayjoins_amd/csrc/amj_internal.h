@@ -103,7 +103,7 @@ struct Plan {
   const int32_t* sfx_base;            // suffix table: column k at sfx_base + k * sfx_stride
   uint64_t sfx_stride;
   int32_t sfx_cols;                   // columns of the suffix table (0..kMaxAttrs)
-  int32_t pad2;
+  int32_t probe_sfx;                  // 1: the suffix rows of a probe record are [pad, pad + val)
 };
 
 // ---------------------------------------------------------------------------------------

@@ -24,39 +24,23 @@ namespace amj {
 
 constexpr uint64_t kDefaultWindow = 4096;  // results per window of the output-window writer
 
-// One launch of the output-window writer over plan Q; returns AMJ_ERR_STATE on overflow.
+// One launch of the output-window writer over plan Q, into the overflow flag of the query
+// (cleared by the caller).
 static int window_pass(amj_ctx_t* ctx, const Plan& Q, const uint64_t* off, uint64_t total,
-                       const ProbeOut& out, bool hash, uint64_t window, uint64_t* csum,
-                       double* kernel_ms) {
+                       const ProbeOut& out, bool hash, uint64_t window, uint32_t* flag) {
   hipStream_t s = ctx->stream;
-  if (total == 0) {
-    if (csum) *csum = 0;
-    return AMJ_OK;
-  }
+  if (total == 0) return AMJ_OK;
   const uint64_t n_windows = (total + window - 1) / window;
   const uint64_t nb = window_blocks(total, window);
-  void *bsum = nullptr, *first = nullptr, *flag = nullptr;
+  void *bsum = nullptr, *first = nullptr;
   AMJ_TRY(scratch(ctx, SLOT_BLOCK_SUMS, (nb + 1) * 8, &bsum));
   AMJ_TRY(scratch(ctx, SLOT_MISC0, (n_windows + 1) * 8, &first));
-  AMJ_TRY(scratch(ctx, SLOT_FLAG, 256, &flag));
-  AMJ_HIP_TRY(ctx, hipMemsetAsync(flag, 0, 4, s));
   uint64_t nb_used = 0;
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[3], s));
   AMJ_HIP_TRY(ctx, launch_window_write(Q, off, (uint64_t*)first, total, window, out, hash,
-                                       (uint64_t*)bsum, (uint32_t*)flag, &nb_used, s));
+                                       (uint64_t*)bsum, flag, &nb_used, s));
   AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[4], s));
-  uint32_t overflow = 0;
-  AMJ_HIP_TRY(ctx, hipMemcpyAsync(&overflow, flag, 4, hipMemcpyDeviceToHost, s));
-  if (hash && csum) {
-    AMJ_TRY(finish_checksum(ctx, (const uint64_t*)bsum, nb_used, csum));
-  } else {
-    AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
-  }
-  if (kernel_ms) *kernel_ms = elapsed_ms(ctx->ev[3], ctx->ev[4]);
-  if (overflow) {
-    set_error(ctx, AMJ_ERR_STATE, "a frontier level exceeded 2^32 children");
-    return AMJ_ERR_STATE;
-  }
+  if (hash) AMJ_TRY(enqueue_totals(ctx, (const uint64_t*)bsum, nullptr, nb_used));
   return AMJ_OK;
 }
 
@@ -113,7 +97,8 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
     AMJ_TRY(scratch(ctx, SLOT_FIB_W, (n + 1) * 8, &w));
     AMJ_TRY(scratch(ctx, SLOT_SCAN_TEMP, scan_temp_elems(n + 1) * 8, &tmp));
     AMJ_HIP_TRY(ctx, launch_fib_weights(P, t, (uint64_t*)w, (RunRef*)nx, s));
-    AMJ_HIP_TRY(ctx, exclusive_scan_u64((uint64_t*)w, (uint64_t*)p, n + 1, (uint64_t*)tmp, s));
+    AMJ_HIP_TRY(ctx, exclusive_scan_u64((uint64_t*)w, (uint64_t*)p, n + 1, (uint64_t*)tmp, s,
+                                        ctx->mail + MAIL_FIB + 1 + t));
     pw[t] = (uint64_t*)p;
     rec[t] = (RunRef*)nx;
     P.tab[t].pw = pw[t];
@@ -125,15 +110,14 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
   AMJ_TRY(scratch(ctx, SLOT_FIB_W, (n0 + 1) * 8, &w));
   AMJ_TRY(scratch(ctx, SLOT_SCAN_TEMP, scan_temp_elems(n0 + 1) * 8, &tmp));
   AMJ_HIP_TRY(ctx, launch_fib_probe_weights(P, (uint64_t*)w, (RunRef*)pnx, s));
-  AMJ_HIP_TRY(ctx, exclusive_scan_u64((uint64_t*)w, (uint64_t*)off, n0 + 1, (uint64_t*)tmp, s));
+  AMJ_HIP_TRY(ctx, exclusive_scan_u64((uint64_t*)w, (uint64_t*)off, n0 + 1, (uint64_t*)tmp, s,
+                                      ctx->mail + MAIL_FIB));
 
   // sizes: total results and |S_t| for every table
-  uint64_t total = 0;
   uint64_t srows[kMaxLevels] = {0};
-  AMJ_HIP_TRY(ctx, hipMemcpyAsync(&total, (uint64_t*)off + n0, 8, hipMemcpyDeviceToHost, s));
-  for (int t = 0; t <= L - 2; ++t)
-    AMJ_HIP_TRY(ctx, hipMemcpyAsync(&srows[t], pw[t] + P.tab[t].n, 8, hipMemcpyDeviceToHost, s));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(s));
+  const uint64_t total = mail_word(ctx, MAIL_FIB);
+  for (int t = 0; t <= L - 2; ++t) srows[t] = mail_word(ctx, MAIL_FIB + 1 + t);
   srows[L - 1] = P.tab[L - 1].n;
   res->count = total;
 
@@ -157,13 +141,17 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
     }
   }
 
-  // 3. records that lead into a materialised suffix table address its rows
+  // 3. records that lead into a materialised suffix table address its rows (probe records hold
+  // both runs)
   for (int t = L - 3; t >= 0 && t >= k - 1; --t)
     AMJ_HIP_TRY(ctx, launch_records_to_suffix(rec[t], P.tab[t].n, pw[t + 1], s));
-  if (k == 0 && L >= 2)
-    AMJ_HIP_TRY(ctx, launch_records_to_suffix((RunRef*)pnx, n0, pw[0], s));
 
-  // 4. suffix tables, bottom-up
+  // 4. suffix tables, bottom-up. Their writers and the result's run back to back: one that
+  // overflows leaves rows of its table unwritten, which the next ones copy but never use as an
+  // index, and the flag is read once at the end.
+  void* flag = nullptr;
+  AMJ_TRY(scratch(ctx, SLOT_FLAG, 256, &flag));
+  AMJ_HIP_TRY(ctx, hipMemsetAsync(flag, 0, 4, s));
   const int32_t* sbase[kMaxLevels];
   uint64_t sstride[kMaxLevels];
   sbase[L - 1] = P.tab[L - 1].vals;
@@ -174,7 +162,8 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
                               : kDefaultWindow;
   for (int t = L - 2; t >= k; --t) {
     void* buf = nullptr;
-    AMJ_TRY(scratch(ctx, SLOT_SFX0 + t, std::max<uint64_t>(srows[t], 1) * ncols[t] * 4, &buf));
+    sstride[t] = (srows[t] + kColAlign - 1) / kColAlign * kColAlign;
+    AMJ_TRY(scratch(ctx, SLOT_SFX0 + t, std::max<uint64_t>(sstride[t], 1) * ncols[t] * 4, &buf));
     Plan Q;
     std::memset(&Q, 0, sizeof(Q));
     Q.n_levels = 1;
@@ -188,11 +177,10 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
     Q.sfx_stride = sstride[t + 1];
     Q.sfx_cols = ncols[t + 1];
     ProbeOut po{};
-    for (int a = 0; a < ncols[t]; ++a) po.cols[a] = (int32_t*)buf + (uint64_t)a * srows[t];
+    for (int a = 0; a < ncols[t]; ++a) po.cols[a] = (int32_t*)buf + (uint64_t)a * sstride[t];
     po.capacity = srows[t];
-    AMJ_TRY(window_pass(ctx, Q, pw[t], srows[t], po, false, window, nullptr, nullptr));
+    AMJ_TRY(window_pass(ctx, Q, pw[t], srows[t], po, false, window, (uint32_t*)flag));
     sbase[t] = (const int32_t*)buf;
-    sstride[t] = srows[t];
   }
 
   // 5. the result: top levels 0..k-1 traversed, last hop into S_k
@@ -203,6 +191,7 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
   F.sfx_base = sbase[k];
   F.sfx_stride = sstride[k];
   F.sfx_cols = ncols[k];
+  F.probe_sfx = k == 0 && L >= 2;
   ProbeOut out{};
   if (o->materialize && total > 0) {
     if (out_bytes > budget_left(ctx, o)) {
@@ -216,17 +205,26 @@ int run_fib(amj_ctx_t* ctx, const Plan& plan, const amj_opts_t* o, amj_result_t*
     out.capacity = total;
   }
   const bool hash = o->checksum || !out.cols[0];
-  double kms = 0.0;
-  const int rc = window_pass(ctx, F, (const uint64_t*)off, total, out, hash, window,
-                             hash ? &res->checksum : nullptr, &kms);
+  ctx->mail[MAIL_FIB] = 0;
+  const auto run = [&]() -> int {
+    AMJ_TRY(window_pass(ctx, F, (const uint64_t*)off, total, out, hash, window, (uint32_t*)flag));
+    AMJ_HIP_TRY(ctx, hipMemcpyAsync(ctx->mail + MAIL_FIB, flag, 4, hipMemcpyDeviceToHost, s));
+    AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[5], s));
+    AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[5]));
+    return AMJ_OK;
+  };
+  int rc = run();
+  if (rc == AMJ_OK && mail_word(ctx, MAIL_FIB) != 0) {
+    set_error(ctx, AMJ_ERR_STATE, "a frontier level exceeded 2^32 children");
+    rc = AMJ_ERR_STATE;
+  }
   if (rc != AMJ_OK) {
     amj_result_free(ctx, res);
     return rc;
   }
-  AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[5], s));
-  AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[5]));
+  if (hash) res->checksum = total > 0 ? mail_word(ctx, MAIL_TOTALS) : 0;
   res->probe_ms = elapsed_ms(ctx->ev[2], ctx->ev[5]);
-  res->probe_kernel_ms = kms;
+  res->probe_kernel_ms = total > 0 ? elapsed_ms(ctx->ev[3], ctx->ev[4]) : 0.0;
   res->probe_kernel_launches = 1;
   res->rows_written = out.cols[0] ? total : 0;
   res->path = AMJ_PATH_FIB;

@@ -512,15 +512,19 @@ int alloc_output(amj_ctx_t* ctx, uint64_t rows, int n_attrs, amj_result_t* res) 
     ctx->out_pool.erase(ctx->out_pool.begin() + pick);
     ctx->pool_bytes -= got;
   } else {
-    int rc = dmalloc(ctx, &base, bytes);
-    if (rc == AMJ_ERR_NOMEM && !ctx->out_pool.empty()) {
+    got = std::max<uint64_t>((rows + kColAlign - 1) / kColAlign * kColAlign, 1) *
+          sizeof(int32_t) * (size_t)n_attrs;
+    int rc = dmalloc(ctx, &base, got);
+    if (rc == AMJ_ERR_NOMEM) {
       pool_clear(ctx);
-      rc = dmalloc(ctx, &base, bytes);
+      got = bytes;
+      rc = dmalloc(ctx, &base, got);
     }
     if (rc != AMJ_OK) return rc;
-    got = bytes;
   }
-  const uint64_t per_col = got / sizeof(int32_t) / (size_t)n_attrs;
+  uint64_t per_col = got / sizeof(int32_t) / (size_t)n_attrs;
+  // columns start at whole cache lines where there is room (see flush_full_block)
+  if (per_col / kColAlign * kColAlign >= rows) per_col = per_col / kColAlign * kColAlign;
   for (int a = 0; a < n_attrs; ++a) res->cols[a] = (int32_t*)base + (uint64_t)a * per_col;
   res->reserved[0] = (uint32_t)(got & 0xffffffffu);
   res->reserved[1] = (uint32_t)(got >> 32);

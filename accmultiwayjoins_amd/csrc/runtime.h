@@ -186,6 +186,7 @@ double elapsed_ms(hipEvent_t a, hipEvent_t b);
 
 // Helpers shared by the execution drivers (runtime.cpp, fib.cpp).
 bool fib_eligible(const Plan& P);
+constexpr uint64_t kColAlign = 64;  // rows between possible starts of a result's columns
 int alloc_output(amj_ctx_t* ctx, uint64_t rows, int n_attrs, amj_result_t* res);
 int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb, uint64_t* out);
 // Enqueue the sums of nb per-block checksums and (may be nullptr) counts; they are read with

@@ -41,10 +41,13 @@ struct ChainOut {
 };
 
 typedef __attribute__((address_space(3))) int32_t lds_i32;
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+typedef i32x4 i32x4_any __attribute__((aligned(4)));  // columns start at any row
+typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
 
 // Results are staged per wave in an LDS ring of two kBlk-row blocks (column a at
-// stage[a * kStageRows ..]) and leave in whole blocks: per column, kBlk / 64 stores of 256
-// aligned bytes issued back to back, so each column receives 1 KB at a time. Measured against
+// stage[a * kStageRows ..]) and leave in whole blocks, 1 KB of a column at a time. Measured (with
+// 4-byte stores) against
 // 64-row blocks: 21.9-23.2 ms against 23.1-23.8 ms for the 2^32-result chain on one box,
 // 24.5-24.7 against 26.5 ms on another (fewer, longer runs of writes per column; a ring of
 // kBlk + 64 rows, which leaves room for one more wave per SIMD, was slower). Windows start at
@@ -85,18 +88,21 @@ __device__ __forceinline__ void flush_block(const ChainOut& out, lds_i32* stage,
 }
 
 // Write the complete block b of the staging ring (no lane predicate, so the compiler knows the
-// wave issues exactly NA * kBlk / 64 stores).
+// wave issues exactly NA stores): one store of 16 B per lane and column, 1 KB in a row, past the
+// caches. The writer is bound by its stores: 1.07 G results of 5 columns (21.5 GB) took 6.55 ms
+// with four 4-byte stores per lane and column, 6.03 with one of 16 B, 5.50 with the columns
+// starting at whole cache lines (alloc_output) and 5.23 with nontemporal stores; hashing the same
+// results without output takes 1.9.
 template <int NA>
 __device__ __forceinline__ void flush_full_block(const ChainOut& out, lds_i32* stage,
                                                  uint64_t b) {
+  static_assert(kBlk == 4 * kWave, "four rows per lane");
   __asm__ __volatile__("" ::: "memory");  // LDS ops of one wave complete in order
-  const uint32_t lane = (uint32_t)lane_id();
+  const uint64_t row = b * kBlk + 4u * (uint32_t)lane_id();
+  const uint32_t slot = (uint32_t)row & (kStageRows - 1);
   sfor<0, NA>([&](auto a) {
-    sfor<0, kBlk / kWave>([&](auto k) {
-      const uint64_t row = b * kBlk + (uint32_t)k * kWave + lane;
-      const uint32_t slot = (uint32_t)row & (kStageRows - 1);
-      out.base[(uint64_t)a * out.stride + row] = stage[a * kStageRows + slot];
-    });
+    const i32x4 v = *(const lds_i32x4*)(stage + a * kStageRows + slot);
+    __builtin_nontemporal_store(v, (i32x4_any*)(out.base + (uint64_t)a * out.stride + row));
   });
   __asm__ __volatile__("" ::: "memory");
 }
@@ -111,11 +117,20 @@ __device__ __forceinline__ bool finish_w(ChainLv<NB>& l) {
   return true;
 }
 
-template <int NA>
-__device__ __forceinline__ uint64_t hash_chain(const int32_t (&v)[NA]) {
-  int32_t w[kMaxAttrs];
-  sfor<0, kMaxAttrs>([&](auto a) { w[a] = (a < NA) ? v[(a < NA) ? (int)a : 0] : 0; });
-  return hash_tuple(w, NA);
+// Rounds [J0, J1) of the hash of an NA-value tuple (hash_tuple's rounds: pairs of attributes)
+// from h, over its first N values. The rounds whose values an entry of the last level holds are
+// done once per entry and not per result: a round is two 64-bit multiplies, several times the two
+// shuffles that fetch its state (1.07 G five-value results counted and hashed: 2.44 -> 1.86 ms).
+template <int NA, int J0, int J1, int N>
+__device__ __forceinline__ uint64_t hash_rounds(uint64_t h, const int32_t (&v)[N]) {
+  static_assert(J1 == (NA + 1) / 2 || 2 * J1 <= N, "the rounds' values are there");
+  sfor<J0, J1>([&](auto j) {
+    constexpr int i = 2 * (int)j;
+    uint64_t hi = 0;
+    if constexpr (i + 1 < NA) hi = (uint64_t)(uint32_t)v[i + 1] << 32;
+    h = mix64(h ^ ((uint64_t)(uint32_t)v[i] | hi));
+  });
+  return h;
 }
 
 // L frontier levels: level 0 = probe rows, level t = rows of table t-1; the children of level
@@ -136,9 +151,10 @@ struct Chain {
       sfor<0, PC>([&](auto c) { l.b[c] = __builtin_nontemporal_load(&P.probe_cols[c][r]); });
       rr = P.probe_next[r];
     }
-    l.len = rr.len;
+    const bool sfx = L == 1 && P.probe_sfx;
+    l.len = sfx ? (uint32_t)rr.val : rr.len;
     const bool ok = finish_w(l);
-    l.base = rr.lo - l.excl;
+    l.base = (sfx ? rr.pad : rr.lo) - l.excl;
     return ok;
   }
 
@@ -200,6 +216,12 @@ struct Chain {
                                               AccW& acc) {
     const int32_t* sfx = P.sfx_base;
     const uint64_t sst = P.sfx_stride;
+    constexpr int kPre = NB / 2;  // hash rounds an entry's own bindings fill
+    const uint64_t pre = HASH ? hash_rounds<NA, 0, kPre>((uint64_t)NA, l.b) : 0ull;
+    auto hash_of = [&](int p, const int32_t (&v)[NA]) {
+      const uint64_t h = kPre > 0 ? __shfl(pre, p, kWave) : pre;
+      return hash_rounds<NA, kPre, (NA + 1) / 2>(h, v);
+    };
     auto locate = [&](uint32_t c, int& p, int32_t (&sv)[NV > 0 ? NV : 1]) {
       p = (int)parent_of_slots(l.excl, l.len, c);
       const uint32_t g = c + (uint32_t)lane_id();
@@ -214,8 +236,9 @@ struct Chain {
       sfor<0, NB>([&](auto a) { v[a] = __shfl(l.b[a], p, kWave); });
       if constexpr (NV > 0) sfor<0, NV>([&](auto k) { v[NB + k] = sv[k]; });
       const uint32_t g = c + (uint32_t)lane_id();
+      const uint64_t h = HASH ? hash_of(p, v) : 0ull;  // every lane takes part in its shuffle
       if (g < e1) {
-        if (HASH) acc.csum += hash_chain<NA>(v);
+        if (HASH) acc.csum += h;
         if (MAT) {
           const uint32_t slot = (uint32_t)(e0 + g) & (kStageRows - 1);
           sfor<0, NA>([&](auto a) { acc.stage[a * kStageRows + slot] = v[a]; });
@@ -225,7 +248,7 @@ struct Chain {
         const uint32_t m = (e1 - c) < (uint32_t)kWave ? (e1 - c) : (uint32_t)kWave;
         const uint64_t rb = e0 + c, re = rb + m;
         if ((rb >> kLgBlk) != (re >> kLgBlk))
-          flush_block<NA>(out, acc.stage, rb >> kLgBlk, (uint32_t)kBlk);
+          flush_full_block<NA>(out, acc.stage, rb >> kLgBlk);
       }
     };
     constexpr uint32_t GW = (uint32_t)(kEmitGroup * kWave);  // results per group
@@ -246,7 +269,7 @@ struct Chain {
         int32_t v[NA];
         sfor<0, NB>([&](auto a) { v[a] = __shfl(l.b[a], pg[i], kWave); });
         if constexpr (NV > 0) sfor<0, NV>([&](auto k) { v[NB + k] = sg[i][k]; });
-        if (HASH) acc.csum += hash_chain<NA>(v);
+        if (HASH) acc.csum += hash_of(pg[i], v);
         if (MAT) {
           const uint32_t slot = (uint32_t)(e0 + ci + lane_id()) & (kStageRows - 1);
           sfor<0, NA>([&](auto a) { acc.stage[a * kStageRows + slot] = v[a]; });
@@ -311,7 +334,7 @@ __global__ __launch_bounds__(kBlock) void window_write_kernel(
     uint64_t* __restrict__ block_sums, uint32_t* __restrict__ overflow) {
   using C = Chain<L, PC, NV>;
   constexpr int NA = Chain<L, PC, NV>::NA;
-  __shared__ int32_t stage_mem[MAT ? kWavesPerBlock * NA * kStageRows : 1];
+  __shared__ __attribute__((aligned(16))) int32_t stage_mem[MAT ? kWavesPerBlock * NA * kStageRows : 1];
   const uint64_t blk = xcd_block(blockIdx.x, gridDim.x);  // neighbouring windows per XCD
   // windows w, w + n_slots, ...: the grid is capped (a launch holds fewer than 2^32 lanes)
   const uint64_t n_slots = (uint64_t)gridDim.x * kWavesPerBlock;

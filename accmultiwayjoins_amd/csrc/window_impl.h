@@ -47,11 +47,10 @@ typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
 
 // Results are staged per wave in an LDS ring of two kBlk-row blocks (column a at
 // stage[a * kStageRows ..]) and leave in whole blocks, 1 KB of a column at a time. Measured (with
-// 4-byte stores) against
-// 64-row blocks: 21.9-23.2 ms against 23.1-23.8 ms for the 2^32-result chain on one box,
-// 24.5-24.7 against 26.5 ms on another (fewer, longer runs of writes per column; a ring of
-// kBlk + 64 rows, which leaves room for one more wave per SIMD, was slower). Windows start at
-// multiples of kBlk rows, so a block never straddles two waves.
+// 4-byte stores) against 64-row blocks: 21.9-23.2 ms against 23.1-23.8 ms for the 2^32-result
+// chain on one box, 24.5-24.7 against 26.5 ms on another (fewer, longer runs of writes per column;
+// a ring of kBlk + 64 rows, which leaves room for one more wave per SIMD, was slower). Windows
+// start at multiples of kBlk rows, so a block never straddles two waves.
 constexpr int kBlk = 256;
 constexpr int kLgBlk = 8;
 constexpr int kStageRows = 2 * kBlk;

@@ -59,8 +59,6 @@ struct DevTable {
   const int32_t* keys;    // [n] hash-column values, bucket-major
   const int32_t* vals;    // [n] second-column values in the same order (nullptr: 1 column)
   const uint64_t* pw;     // [n+1] exclusive prefix of subtree weights (frequent-item buffer)
-  const uint4* rec;       // [B] {first row, end, first key, last key} of each bucket (nullptr:
-                          // none; identity tables need none)
   uint64_t n;
   uint32_t log_b;
   uint32_t identity;      // every key lies in [0, B): bucket b holds only key b
@@ -226,21 +224,20 @@ struct HashTableDev {
   int32_t* keys = nullptr;
   int32_t* vals = nullptr;
   uint64_t* pw = nullptr;
-  uint4* rec = nullptr;
   uint64_t buckets = 0;
 };
 
 // Launch helpers used by the host runtime.
 hipError_t launch_bucket_ptrs(const uint64_t* comp, uint64_t n, uint32_t log_b,
                               uint64_t buckets, uint32_t* ptrs, hipStream_t s);
-// Bucket pointers and (rec != nullptr) records of bucket-sorted keys; n > 0.
+// Bucket pointers of bucket-sorted keys; n > 0.
 hipError_t launch_bucket_index(const int32_t* keys, uint64_t n, uint64_t buckets, uint32_t* ptrs,
-                               uint4* rec, hipStream_t s);
-// The whole build of at most kHashSmallRows rows (c as for launch_col_sort, buf_x and buf_y
+                               hipStream_t s);
+// The whole build of at most kHashSmallRows rows (c as for run_col_sort, buf_x and buf_y
 // unused), the key-range flag included.
 constexpr uint64_t kHashSmallRows = 8192;
 struct ColSort;
-hipError_t launch_hash_small(const ColSort& c, uint32_t log_b, uint32_t* ptrs, uint4* rec,
+hipError_t launch_hash_small(const ColSort& c, uint32_t log_b, uint32_t* ptrs,
                              uint32_t* flag_out, hipStream_t s);
 
 // ---------------------------------------------------------------------------------------

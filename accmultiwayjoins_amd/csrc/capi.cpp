@@ -257,11 +257,6 @@ void amj_hash_table_destroy(amj_ctx_t* ctx, amj_hash_table_t* ht) {
   dfree(ctx, ht->dev.ptrs, (ht->dev.buckets + 1) * 4);
   dfree(ctx, ht->dev.keys, n * 4);
   dfree(ctx, ht->dev.vals, n * 4);
-  if (ht->dev.rec) {
-    const uint64_t rec = ht->dev.buckets * sizeof(uint4);
-    dfree(ctx, ht->dev.rec, rec);
-    if (ctx) ctx->rec_bytes -= std::min(ctx->rec_bytes, rec);
-  }
   delete ht;
 }
 

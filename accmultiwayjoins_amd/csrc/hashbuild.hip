@@ -20,14 +20,6 @@
 
 namespace amj {
 
-// One 16-byte record per bucket (DevTable::rec): first row, end, first and last key. With it a
-// lookup in a table whose keys lie past its buckets is one load where it was two dependent ones
-// over three cache lines (bucket pointers, then the bucket's first and last key).
-__device__ __forceinline__ uint4 bucket_record(const int32_t* keys, uint32_t s, uint32_t e) {
-  return s < e ? make_uint4(s, e, (uint32_t)keys[s], (uint32_t)keys[e - 1])
-               : make_uint4(s, s, 0u, 0u);
-}
-
 // First row of [0, n) whose bucket is >= b, found by a whole wave: 64 positions per step, so four
 // dependent loads for 16 M rows.
 __device__ __forceinline__ uint64_t wave_lower_bucket(const int32_t* __restrict__ keys, uint64_t n,
@@ -46,8 +38,7 @@ __device__ __forceinline__ uint64_t wave_lower_bucket(const int32_t* __restrict_
   return lo;
 }
 
-// Bucket pointers (ptrs[b] = first row whose bucket is >= b, ptrs[B] = n) and records of the sorted
-// keys. A workgroup takes kIdxBuckets consecutive buckets: it finds their rows, reads those keys
+// Bucket pointers of the sorted keys: ptrs[b] = first row whose bucket is >= b, ptrs[B] = n. A workgroup takes kIdxBuckets consecutive buckets: it finds their rows, reads those keys
 // once, in order, notes the first row of every bucket present in LDS, and a suffix minimum over
 // the buckets fills the empty ones. A workgroup whose buckets hold more than kIdxScanRows
 // rows (a heavy key) searches each bucket's bound instead, so no workgroup reads a long run. One
@@ -58,9 +49,8 @@ constexpr uint32_t kIdxItems = kIdxBuckets / kBlock;
 constexpr uint64_t kIdxScanRows = 16 * kIdxBuckets;
 __global__ __launch_bounds__(kBlock) void bucket_index_kernel(const int32_t* __restrict__ keys,
                                                               uint64_t n, uint64_t buckets,
-                                                              uint32_t* __restrict__ ptrs,
-                                                              uint4* __restrict__ rec) {
-  __shared__ uint32_t first[kIdxBuckets + 1];
+                                                              uint32_t* __restrict__ ptrs) {
+  __shared__ uint32_t first[kIdxBuckets];
   __shared__ uint64_t range[2];
   __shared__ uint32_t wave_min[kWavesPerBlock];
   const uint32_t mask = (uint32_t)(buckets - 1);
@@ -117,25 +107,21 @@ __global__ __launch_bounds__(kBlock) void bucket_index_kernel(const int32_t* __r
     after = min(after, v[i]);
     first[tid * kIdxItems + i] = after;
   }
-  if (tid == 0) first[kIdxBuckets] = (uint32_t)r1;
   __syncthreads();
   for (uint32_t i = tid; i < nb; i += kBlock) ptrs[b0 + i] = first[i];
-  if (rec)
-    for (uint32_t i = tid; i < nb; i += kBlock)
-      rec[b0 + i] = bucket_record(keys, first[i], first[i + 1]);
   if (b0 + nb == buckets && tid == 0) ptrs[buckets] = (uint32_t)n;
 }
 
 hipError_t launch_bucket_index(const int32_t* keys, uint64_t n, uint64_t buckets, uint32_t* ptrs,
-                               uint4* rec, hipStream_t s) {
+                               hipStream_t s) {
   const uint64_t blocks = (buckets + kIdxBuckets - 1) / kIdxBuckets;
   hipLaunchKernelGGL(bucket_index_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, keys, n,
-                     buckets, ptrs, rec);
+                     buckets, ptrs);
   return hipGetLastError();
 }
 
 // The whole build of a table of up to 1024 * ITEMS rows in one workgroup: rows in registers, every
-// sorting pass through one LDS copy, then the columns, the bucket pointers and the records. Bound
+// sorting pass through one LDS copy, then the columns and the bucket pointers. Bound
 // by the latency of its few passes: 19 us for 4,096 rows, where the tiled build (three kernels per
 // digit and three around them) takes about 90. 8,192 rows are what registers and LDS hold at
 // eight rows per lane.
@@ -143,7 +129,7 @@ constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / kWave;
 template <int ITEMS>
 __global__ __launch_bounds__(kSmallThreads) void hash_small_kernel(
-    const ColSort c, uint32_t log_b, uint32_t* __restrict__ ptrs, uint4* __restrict__ rec,
+    const ColSort c, uint32_t log_b, uint32_t* __restrict__ ptrs,
     uint32_t* __restrict__ flag_out) {
   __shared__ uint64_t tile[kSmallThreads * ITEMS];
   __shared__ uint32_t wrun[kSmallWaves][256];
@@ -233,29 +219,19 @@ __global__ __launch_bounds__(kSmallThreads) void hash_small_kernel(
     }
     return lo;
   };
-  for (uint32_t b = (uint32_t)tid; b < buckets; b += kSmallThreads) {
-    const uint32_t s = lower(b);
-    uint32_t e = s;
-    while (e < n && e - s < 4 && bucket(e) == b) ++e;
-    if (e < n && bucket(e) == b) e = lower(b + 1);
-    ptrs[b] = s;
-    const auto key_at = [&](uint32_t i) {
-      return rotl32((uint32_t)(tile[i] >> 32), c.rot);
-    };
-    rec[b] = s < e ? make_uint4(s, e, key_at(s), key_at(e - 1)) : make_uint4(s, s, 0u, 0u);
-  }
+  for (uint32_t b = (uint32_t)tid; b < buckets; b += kSmallThreads) ptrs[b] = lower(b);
   if (tid == 0) {
     ptrs[buckets] = n;
     *flag_out = any_out ? 1u : 0u;
   }
 }
 
-hipError_t launch_hash_small(const ColSort& c, uint32_t log_b, uint32_t* ptrs, uint4* rec,
+hipError_t launch_hash_small(const ColSort& c, uint32_t log_b, uint32_t* ptrs,
                              uint32_t* flag_out, hipStream_t s) {
   if (c.n == 0 || c.n > kHashSmallRows) return hipErrorInvalidValue;
 #define LAUNCH(I)                                                                               \
   hipLaunchKernelGGL(hash_small_kernel<I>, dim3(1), dim3(kSmallThreads), 0, s, c, log_b, ptrs, \
-                     rec, flag_out)
+                     flag_out)
   if (c.n <= kSmallThreads) LAUNCH(1);
   else if (c.n <= 4 * kSmallThreads) LAUNCH(4);
   else LAUNCH(8);
@@ -264,7 +240,7 @@ hipError_t launch_hash_small(const ColSort& c, uint32_t log_b, uint32_t* ptrs, u
 }
 
 hipError_t launch_small_sort(const ColSort& c, hipStream_t s) {
-  return launch_hash_small(c, 0, nullptr, nullptr, nullptr, s);
+  return launch_hash_small(c, 0, nullptr, nullptr, s);
 }
 
 // Bucket bounds of sorted composites (the pairwise engine's partitions).

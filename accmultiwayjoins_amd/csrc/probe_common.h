@@ -88,13 +88,6 @@ __device__ __forceinline__ void lookup_run(const DevTable& tb, int32_t key, bool
     if (k > mask) return;  // bucket b holds only key b
     s = tb.ptrs[k];
     e = tb.ptrs[k + 1];
-  } else if (tb.rec) {
-    const uint4 r = tb.rec[k & mask];
-    s = r.x;
-    e = r.y;
-    if (s == e || k < r.z || k > r.w) return;
-    if (r.z != k) s = lower_bound_u32(tb.keys, s + 1, e, k);
-    if (r.w != k) e = upper_bound_u32(tb.keys, s, e - 1, k);
   } else {
     const uint32_t b = k & mask;
     s = tb.ptrs[b];

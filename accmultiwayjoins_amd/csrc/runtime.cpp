@@ -147,18 +147,6 @@ int scratch(amj_ctx_t* ctx, int slot, size_t bytes, void** out) {
 // ------------------------------------------------------------------------------------------
 // Hash build.
 // ------------------------------------------------------------------------------------------
-// Bucket records of a table (16 B per bucket), left out (d->rec == nullptr) when they would bring
-// the context's records over an eighth of the device memory or cannot be allocated.
-static int alloc_records(amj_ctx_t* ctx, HashTableDev* d) {
-  const uint64_t bytes = d->buckets * sizeof(uint4);
-  d->rec = nullptr;
-  if (bytes > (1ull << 20) && ctx->rec_bytes + bytes > (uint64_t)ctx->props.totalGlobalMem / 8)
-    return AMJ_OK;
-  if (dmalloc(ctx, (void**)&d->rec, bytes) == AMJ_OK) ctx->rec_bytes += bytes;
-  else d->rec = nullptr;
-  return AMJ_OK;
-}
-
 int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, int sort_vals,
                      amj_hash_table** out) {
   *out = nullptr;
@@ -208,12 +196,7 @@ int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, 
     c.out_val = d.vals;
     if (n <= kHashSmallRows) {
       uint32_t* flag = (uint32_t*)(ctx->mail + MAIL_KEY_RANGE);
-      AMJ_TRY(alloc_records(ctx, &d));
-      if (!d.rec) {
-        set_error(ctx, AMJ_ERR_NOMEM, "no device memory for the bucket records");
-        return AMJ_ERR_NOMEM;
-      }
-      AMJ_HIP_TRY(ctx, launch_hash_small(c, log_b, d.ptrs, d.rec, flag, s));
+      AMJ_HIP_TRY(ctx, launch_hash_small(c, log_b, d.ptrs, flag, s));
       AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[1], s));
       AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[1]));
       identity = *(volatile uint32_t*)flag == 0 ? 1u : 0u;
@@ -226,10 +209,8 @@ int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, 
       c.buf_y = (uint64_t*)y;
       ColSortFacts facts;
       AMJ_HIP_TRY(ctx, run_col_sort(c, tmp, ctx->mail + MAIL_SORT, ctx->ev[6], s, &facts));
-      // known while the device sorts: only tables that are not "identity" have records
       identity = facts.past_limit ? 0u : 1u;
-      if (!identity) AMJ_TRY(alloc_records(ctx, &d));
-      AMJ_HIP_TRY(ctx, launch_bucket_index(d.keys, n, buckets, d.ptrs, d.rec, s));
+      AMJ_HIP_TRY(ctx, launch_bucket_index(d.keys, n, buckets, d.ptrs, s));
       AMJ_HIP_TRY(ctx, hipEventRecord(ctx->ev[1], s));
       AMJ_HIP_TRY(ctx, hipEventSynchronize(ctx->ev[1]));
     }
@@ -244,7 +225,6 @@ int build_hash_table(amj_ctx_t* ctx, const amj_relation* rel, uint32_t key_col, 
   d.view.keys = d.keys;
   d.view.vals = d.vals;
   d.view.pw = nullptr;
-  d.view.rec = identity ? nullptr : d.rec;
   d.view.n = n;
   d.view.log_b = log_b;
   d.view.identity = identity;
@@ -553,8 +533,7 @@ uint64_t budget_left(amj_ctx_t* ctx, const amj_opts_t* o) {
   uint64_t left = free_b + ctx->pool_bytes + ctx->parked_bytes;  // given back when needed
   if (ctx->arena.base) left = arena_largest(ctx);
   if (o && o->hbm_budget_bytes) {
-    const uint64_t held = budget_held(ctx);
-    const uint64_t cap = o->hbm_budget_bytes > held ? o->hbm_budget_bytes - held : 0;
+    const uint64_t cap = o->hbm_budget_bytes > ctx->allocated ? o->hbm_budget_bytes - ctx->allocated : 0;
     left = std::min<uint64_t>(left, cap);
   }
   return left;

@@ -19,7 +19,6 @@ struct amj_ctx {
   uint64_t peak = 0;
   hipEvent_t ev[8]{};
   uint64_t* mail = nullptr;    // pinned host memory that kernels leave small results in
-  uint64_t rec_bytes = 0;      // of `allocated`: bucket records of hash tables (DevTable::rec)
 
   // Reusable scratch buffers keyed by purpose.
   struct Buf {
@@ -149,10 +148,6 @@ enum MailWord {
   MAIL_FIB = 16,       // kMaxLevels + 1 words
   MAIL_WORDS = 64
 };
-
-// Bytes that hbm_budget_bytes counts as held: the bucket records, which only speed lookups up and
-// are not built when memory is short, are not among them.
-inline uint64_t budget_held(const amj_ctx_t* ctx) { return ctx->allocated - ctx->rec_bytes; }
 
 // A table as used by one query: the same physical table may be used several times with
 // different attribute ids (the TRI and FOUR queries alias one edge table).

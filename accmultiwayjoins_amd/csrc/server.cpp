@@ -239,11 +239,11 @@ struct amj_server {
         o.checksum = 1;
         ++c.tuned;
       }
-      o.hbm_budget_bytes = budget_held(ctx) + c.room;
+      o.hbm_budget_bytes = ctx->allocated + c.room;
       if (rc == AMJ_OK)
         rc = amj_execute(ctx, rels[q.ids[0]].rel, hts.data(), (uint32_t)hts.size(), &o, &res);
     } else {
-      o.hbm_budget_bytes = budget_held(ctx) + c.room;
+      o.hbm_budget_bytes = ctx->allocated + c.room;
       Plan plan;
       std::vector<uint32_t> ids;
       rc = make_pattern_plan(ctx, rels[q.ids[0]].rel, rels[q.ids[0]].ht, q.query, &plan, &ids);
@@ -277,7 +277,7 @@ struct amj_server {
       o.checksum = 1;
       o.dro = q.materialize ? 1 : 0;
       o.ws = q.query == AMJ_QUERY_FOUR && !q.materialize ? 1 : 0;
-      o.hbm_budget_bytes = budget_held(ctx) + c.room;
+      o.hbm_budget_bytes = ctx->allocated + c.room;
       static const uint32_t tri[6] = {0, 1, 1, 2, 0, 2};
       static const uint32_t four[12] = {0, 1, 1, 2, 2, 3, 0, 3, 0, 2, 1, 3};
       static const uint32_t order[4] = {0, 1, 2, 3};

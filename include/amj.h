@@ -160,8 +160,8 @@ int amj_sync(amj_ctx_t* ctx);
 /* Pinned host memory (hipHostMalloc) for relations kept on the host (AMJ_REL_HOST): the
  * out-of-core probe streams it to the device at PCIe rate, overlapped with the probe. */
 int amj_host_alloc(size_t bytes, void** out);
-/* Device bytes held by the context now and at its peak (the HBM budget counts the former, less
- * the bucket records of hash tables). Released blocks that the context keeps for its next
+/* Device bytes held by the context now and at its peak (the HBM budget counts the former).
+ * Released blocks that the context keeps for its next
  * allocations (at most 2 GiB, given back when an allocation fails) are not counted. */
 int amj_memory_info(amj_ctx_t* ctx, uint64_t* allocated, uint64_t* peak);
 void amj_host_free(void* p);

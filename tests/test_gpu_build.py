@@ -1,6 +1,6 @@
 """Hash-table builds at the sizes and key patterns where their variants meet: the one-workgroup
 build (up to 8,192 rows), the tiled sort (4,096-row tiles) and the bucket index (2,048 buckets per
-workgroup, heavy buckets searched), tables with and without bucket records. Every build is read
+workgroup, heavy buckets searched), tables of keys below and past the bucket count. Every build is read
 back through a two-relation join whose rows must come out in exactly the order a stable sort
 gives."""
 import numpy as np

@@ -91,7 +91,7 @@ void amj_batch_destroy(amj_batch_t* b) {
   if (b->cap.exec) (void)hipGraphExecDestroy(b->cap.exec);
   if (b->cap.graph) (void)hipGraphDestroy(b->cap.graph);
   if (!b->cap.bufs.empty()) (void)hipStreamSynchronize(b->ctx->stream);
-  for (auto& x : b->cap.bufs) dfree(b->ctx, x.first, x.second);
+  for (auto& x : b->cap.bufs) dfree(b->ctx, x.first);
   delete b;
 }
 

@@ -91,8 +91,7 @@ int amj_ctx_create(int device, amj_ctx_t** out) {
     return AMJ_ERR_NODEV;
   }
   if (device < 0 || device >= n) return AMJ_ERR_ARG;
-  std::unique_ptr<amj_ctx> ctx(new amj_ctx());
-  ctx->device = device;
+  std::unique_ptr<amj_ctx> ctx(new amj_ctx(device));
   if (hipSetDevice(device) != hipSuccess) return AMJ_ERR_HIP;
   if (hipGetDeviceProperties(&ctx->props, device) != hipSuccess) return AMJ_ERR_HIP;
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
@@ -113,11 +112,9 @@ void amj_ctx_destroy(amj_ctx_t* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   (void)hipDeviceSynchronize();
-  ctx->closing = true;
-  park_clear(ctx);
-  for (auto& kv : ctx->scratch) dfree(ctx, kv.second.p, kv.second.bytes);
+  for (auto& kv : ctx->scratch) ctx->blocks.give(kv.second.p, false);
   pool_clear(ctx);
-  if (ctx->arena.base) dfree(ctx, ctx->arena.base, ctx->arena.size);
+  ctx->blocks.give(ctx->arena.base, false);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
   if (ctx->mail) (void)hipHostFree(ctx->mail);
@@ -147,8 +144,8 @@ void amj_host_free(void* p) {
 
 int amj_memory_info(amj_ctx_t* ctx, uint64_t* allocated, uint64_t* peak) {
   if (!ctx) return AMJ_ERR_ARG;
-  if (allocated) *allocated = ctx->allocated;
-  if (peak) *peak = ctx->peak;
+  if (allocated) *allocated = ctx->blocks.held();
+  if (peak) *peak = ctx->blocks.peak();
   return AMJ_OK;
 }
 
@@ -225,7 +222,7 @@ int amj_relation_create(amj_ctx_t* ctx, const amj_rel_t* r, amj_relation_t** out
       }
     }
     if (rc != AMJ_OK) {
-      dfree(ctx, rel->cols[0], step * r->num_cols);
+      dfree(ctx, rel->cols[0]);
       return rc;
     }
   } else {
@@ -239,7 +236,7 @@ void amj_relation_destroy(amj_ctx_t* ctx, amj_relation_t* rel) {
   if (!rel) return;
   if (rel->owned) {
     if (ctx) (void)hipStreamSynchronize(ctx->stream);
-    dfree(ctx, rel->cols[0], owned_col_bytes(rel->rows) * rel->num_cols);
+    dfree(ctx, rel->cols[0]);
   }
   delete rel;
 }
@@ -253,10 +250,9 @@ int amj_hash_table_build(amj_ctx_t* ctx, const amj_relation_t* rel, uint32_t key
 void amj_hash_table_destroy(amj_ctx_t* ctx, amj_hash_table_t* ht) {
   if (!ht) return;
   if (ctx) (void)hipStreamSynchronize(ctx->stream);
-  const uint64_t n = std::max<uint64_t>(ht->dev.view.n, 1);
-  dfree(ctx, ht->dev.ptrs, (ht->dev.buckets + 1) * 4);
-  dfree(ctx, ht->dev.keys, n * 4);
-  dfree(ctx, ht->dev.vals, n * 4);
+  dfree(ctx, ht->dev.ptrs);
+  dfree(ctx, ht->dev.keys);
+  dfree(ctx, ht->dev.vals);
   delete ht;
 }
 

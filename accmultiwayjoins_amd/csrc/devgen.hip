@@ -196,7 +196,7 @@ struct GenBufs {
   explicit GenBufs(amj_ctx_t* c) : ctx(c) {}
   ~GenBufs() {
     if (!held.empty()) (void)hipStreamSynchronize(ctx->stream);
-    for (auto& h : held) dfree(ctx, h.first, h.second);
+    for (auto& h : held) dfree(ctx, h.first);
   }
   int get(size_t bytes, void** p) {
     AMJ_TRY(dmalloc(ctx, p, bytes ? bytes : 8));
@@ -230,7 +230,8 @@ int amj_device_alloc(amj_ctx_t* ctx, size_t bytes, void** out) {
 void amj_device_free(amj_ctx_t* ctx, void* p, size_t bytes) {
   if (!ctx || !p) return;
   (void)hipDeviceSynchronize();  // the caller's work on it may be on streams of its own
-  dfree(ctx, p, bytes ? bytes : 1);
+  (void)bytes;  // the context knows it
+  dfree(ctx, p);
 }
 
 int amj_memcpy(amj_ctx_t* ctx, void* dst, const void* src, size_t bytes) {

@@ -203,7 +203,7 @@ static int grow(amj_ctx_t* ctx, GrowBuf& b, size_t need, size_t keep_bytes) {
   if (b.p && keep_bytes)
     AMJ_HIP_TRY(ctx, hipMemcpyAsync(q, b.p, keep_bytes, hipMemcpyDeviceToDevice, ctx->stream));
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  dfree(ctx, b.p, b.bytes);
+  dfree(ctx, b.p);
   b.p = q;
   b.bytes = want;
   return AMJ_OK;
@@ -219,7 +219,7 @@ static int bfs_run(amj_ctx_t* ctx, const LPlan& P, uint64_t budget, uint64_t* co
   int rc = AMJ_OK;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    for (GrowBuf* b : {&cur, &nxt, &tmp, &keep, &pos, &len}) dfree(ctx, b->p, b->bytes);
+    for (GrowBuf* b : {&cur, &nxt, &tmp, &keep, &pos, &len}) dfree(ctx, b->p);
   };
   void* stmp = nullptr;
   uint64_t total = 0, csum = 0;

@@ -163,7 +163,7 @@ struct PwBufs {
   explicit PwBufs(amj_ctx_t* c) : ctx(c) {}
   ~PwBufs() {
     if (!held.empty()) (void)hipStreamSynchronize(ctx->stream);
-    for (auto& h : held) dfree(ctx, h.first, h.second);
+    for (auto& h : held) dfree(ctx, h.first);
   }
   template <typename T>
   int get(uint64_t n, T** p) {
@@ -178,7 +178,7 @@ struct PwBufs {
     for (size_t x = 0; x < held.size(); ++x)
       if (held[x].first == p) {
         (void)hipStreamSynchronize(ctx->stream);
-        dfree(ctx, held[x].first, held[x].second);
+        dfree(ctx, held[x].first);
         held.erase(held.begin() + x);
         return;
       }

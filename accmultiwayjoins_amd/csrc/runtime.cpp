@@ -26,72 +26,18 @@ double elapsed_ms(hipEvent_t a, hipEvent_t b) {
   return (double)ms;
 }
 
-// Bytes allocated for a request: classes an eighth of a power of two apart, so that sizes that
-// differ a little share parked blocks.
-static size_t block_bytes(size_t bytes) {
-  if (bytes == 0) bytes = 256;
-  if (bytes > kParkBlock) return bytes;
-  size_t g = 256;
-  while (g * 16 < bytes) g <<= 1;
-  return (bytes + g - 1) / g * g;
-}
-
-void park_clear(amj_ctx_t* ctx) {
-  for (auto& b : ctx->parked) (void)hipFree(b.p);
-  ctx->parked.clear();
-  ctx->parked_bytes = 0;
-}
-
 int dmalloc(amj_ctx_t* ctx, void** p, size_t bytes) {
-  *p = nullptr;
-  const size_t size = block_bytes(bytes);
-  for (size_t i = ctx->parked.size(); i-- > 0;)
-    if (ctx->parked[i].bytes == size) {
-      *p = ctx->parked[i].p;
-      ctx->parked.erase(ctx->parked.begin() + (std::ptrdiff_t)i);
-      ctx->parked_bytes -= size;
-      break;
-    }
-  if (!*p) {
-    hipError_t e = hipMalloc(p, size);
-    if (e != hipSuccess && !(ctx->out_pool.empty() && ctx->parked.empty())) {
-      (void)hipGetLastError();  // parked blocks and result buffers give way first
-      pool_clear(ctx);
-      park_clear(ctx);
-      e = hipMalloc(p, size);
-    }
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      *p = nullptr;
-      set_error(ctx, AMJ_ERR_NOMEM,
-                "hipMalloc(" + std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
-      return AMJ_ERR_NOMEM;
-    }
-  }
-  ctx->allocated += bytes ? bytes : 256;
-  ctx->peak = std::max(ctx->peak, ctx->allocated);
-  return AMJ_OK;
+  const int rc = ctx->blocks.take(bytes, p, [&] { pool_clear(ctx); });
+  if (rc == 0) return AMJ_OK;
+  set_error(ctx, AMJ_ERR_NOMEM, "hipMalloc(" + std::to_string(bytes) +
+                                    " bytes) failed: " + hipGetErrorString((hipError_t)rc));
+  return AMJ_ERR_NOMEM;
 }
 
-static void release_block(amj_ctx_t* ctx, void* p, size_t bytes, bool park) {
-  if (!p) return;
-  const size_t size = block_bytes(bytes);
-  if (ctx) ctx->allocated -= std::min<uint64_t>(ctx->allocated, bytes ? bytes : 256);
-  if (!ctx || !park || ctx->closing || size > kParkBlock) {
-    (void)hipFree(p);
-    return;
-  }
-  ctx->parked.push_back(amj_ctx::Buf{p, size});
-  ctx->parked_bytes += size;
-  while (ctx->parked_bytes > kParkTotal || ctx->parked.size() > kParkCount) {
-    const amj_ctx::Buf b = ctx->parked.front();
-    ctx->parked.erase(ctx->parked.begin());
-    ctx->parked_bytes -= b.bytes;
-    (void)hipFree(b.p);
-  }
+void dfree(amj_ctx_t* ctx, void* p) {
+  if (ctx) ctx->blocks.give(p, true);
+  else if (p) HipDevice{}.put(p);
 }
-
-void dfree(amj_ctx_t* ctx, void* p, size_t bytes) { release_block(ctx, p, bytes, true); }
 
 int stage_upload(amj_ctx_t* ctx, void* dst, const void* const* src, const size_t* at,
                  const size_t* bytes, int n) {
@@ -126,8 +72,10 @@ int scratch(amj_ctx_t* ctx, int slot, size_t bytes, void** out) {
   if (b.bytes < bytes) {
     const size_t old = b.bytes;  // grow by at least half, so growing requests rarely reallocate
     if (b.p) {
+      // the block may be reused at once, also by work on the side stream
       AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-      dfree(ctx, b.p, b.bytes);
+      AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->side));
+      dfree(ctx, b.p);
       b.p = nullptr;
       b.bytes = 0;
     }
@@ -375,12 +323,12 @@ void pool_put(amj_ctx_t* ctx, void* p, size_t bytes) {
     const amj_ctx::Buf b = ctx->out_pool.front();
     ctx->out_pool.erase(ctx->out_pool.begin());
     ctx->pool_bytes -= b.bytes;
-    release_block(ctx, b.p, b.bytes, false);
+    ctx->blocks.give(b.p, false);
   }
 }
 
 void pool_clear(amj_ctx_t* ctx) {
-  for (auto& b : ctx->out_pool) release_block(ctx, b.p, b.bytes, false);
+  for (auto& b : ctx->out_pool) ctx->blocks.give(b.p, false);
   ctx->out_pool.clear();
   ctx->pool_bytes = 0;
 }
@@ -392,7 +340,7 @@ int arena_drop(amj_ctx_t* ctx) {
     return AMJ_ERR_STATE;
   }
   AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  dfree(ctx, ctx->arena.base, ctx->arena.size);
+  dfree(ctx, ctx->arena.base);
   ctx->arena.base = nullptr;
   ctx->arena.size = 0;
   ctx->arena.free.clear();
@@ -530,10 +478,11 @@ int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb, uin
 uint64_t budget_left(amj_ctx_t* ctx, const amj_opts_t* o) {
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-  uint64_t left = free_b + ctx->pool_bytes + ctx->parked_bytes;  // given back when needed
+  uint64_t left = free_b + ctx->pool_bytes + ctx->blocks.parked();  // given back when needed
   if (ctx->arena.base) left = arena_largest(ctx);
   if (o && o->hbm_budget_bytes) {
-    const uint64_t cap = o->hbm_budget_bytes > ctx->allocated ? o->hbm_budget_bytes - ctx->allocated : 0;
+    const uint64_t held = ctx->blocks.held();
+    const uint64_t cap = o->hbm_budget_bytes > held ? o->hbm_budget_bytes - held : 0;
     left = std::min<uint64_t>(left, cap);
   }
   return left;
@@ -628,7 +577,7 @@ struct OaHolder {
   explicit OaHolder(amj_ctx_t* c) : ctx(c) {}
   ~OaHolder() {
     if (!bufs.empty()) (void)hipStreamSynchronize(ctx->stream);
-    for (auto& b : bufs) dfree(ctx, b.first, b.second);
+    for (auto& b : bufs) dfree(ctx, b.first);
   }
   int build(const Plan& P) {
     for (int l = 0; l < P.n_levels; ++l) {

@@ -8,15 +8,31 @@
 #include <vector>
 
 #include "amj_internal.h"
+#include "blocks.h"
+
+namespace amj {
+
+// A context's device, for its Blocks.
+struct HipDevice {
+  int id = 0;
+  int get(size_t bytes, void** p) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return (int)e;
+  }
+  void put(void* p) { (void)hipFree(p); }
+};
+
+}  // namespace amj
 
 struct amj_ctx {
-  int device = 0;
+  explicit amj_ctx(int dev) : device(dev), blocks(amj::HipDevice{dev}) {}
+  const int device;
   hipStream_t stream = nullptr;
   hipStream_t side = nullptr;  // copy stream for out-of-core streaming
   std::string last_error;
   hipDeviceProp_t props{};
-  uint64_t allocated = 0;      // bytes currently allocated by this context
-  uint64_t peak = 0;
+  amj::Blocks<amj::HipDevice> blocks;  // all device memory of the context
   hipEvent_t ev[8]{};
   uint64_t* mail = nullptr;    // pinned host memory that kernels leave small results in
 
@@ -29,11 +45,6 @@ struct amj_ctx {
   // Parked result buffers, reused by later results that fit them (pool_put / alloc_output).
   std::vector<Buf> out_pool;
   uint64_t pool_bytes = 0;
-  // Released device blocks kept for the next allocation of their size (dfree / dmalloc), oldest
-  // first.
-  std::vector<Buf> parked;
-  uint64_t parked_bytes = 0;
-  bool closing = false;
   // Pinned host memory that small columns pass through on their way to or from the device.
   char* staging = nullptr;
   size_t staging_used = 0;  // of it, filled by copies that may still be running
@@ -106,17 +117,9 @@ enum ScratchSlot {
   SLOT_LFTJ_SAMPLE,  // the triejoin's output-size sample: window offsets of the sampled roots
 };
 
-// Device memory. A block of up to kParkBlock bytes is parked when it is released, for a later
-// allocation of its size class (the context's work is in stream order, so it is reused without a
-// wait), at most kParkTotal bytes of them; they are given back when an allocation fails. Allocating
-// and freeing costs 24 us a pair from 4 MB on (260 us for 256 MB), more when the memory has to be
-// cleared first.
-constexpr size_t kParkBlock = 512u << 20;
-constexpr uint64_t kParkTotal = 2ull << 30;
-constexpr size_t kParkCount = 256;
+// Device memory (blocks.h). ctx may be nullptr for dfree: the block goes back to the device.
 int dmalloc(amj_ctx_t* ctx, void** p, size_t bytes);
-void dfree(amj_ctx_t* ctx, void* p, size_t bytes);
-void park_clear(amj_ctx_t* ctx);
+void dfree(amj_ctx_t* ctx, void* p);
 // Columns of up to kStagedCopy bytes are uploaded through the staging buffer: the caller's memory is
 // read before the call returns, the copy is only enqueued. Downloads wait.
 constexpr size_t kStaging = 2u << 20;

@@ -239,11 +239,11 @@ struct amj_server {
         o.checksum = 1;
         ++c.tuned;
       }
-      o.hbm_budget_bytes = ctx->allocated + c.room;
+      o.hbm_budget_bytes = ctx->blocks.held() + c.room;
       if (rc == AMJ_OK)
         rc = amj_execute(ctx, rels[q.ids[0]].rel, hts.data(), (uint32_t)hts.size(), &o, &res);
     } else {
-      o.hbm_budget_bytes = ctx->allocated + c.room;
+      o.hbm_budget_bytes = ctx->blocks.held() + c.room;
       Plan plan;
       std::vector<uint32_t> ids;
       rc = make_pattern_plan(ctx, rels[q.ids[0]].rel, rels[q.ids[0]].ht, q.query, &plan, &ids);
@@ -277,7 +277,7 @@ struct amj_server {
       o.checksum = 1;
       o.dro = q.materialize ? 1 : 0;
       o.ws = q.query == AMJ_QUERY_FOUR && !q.materialize ? 1 : 0;
-      o.hbm_budget_bytes = ctx->allocated + c.room;
+      o.hbm_budget_bytes = ctx->blocks.held() + c.room;
       static const uint32_t tri[6] = {0, 1, 1, 2, 0, 2};
       static const uint32_t four[12] = {0, 1, 1, 2, 2, 3, 0, 3, 0, 2, 1, 3};
       static const uint32_t order[4] = {0, 1, 2, 3};
@@ -590,13 +590,13 @@ int amj_server_memory(amj_server_t* s, uint64_t* resident_bytes, uint64_t* budge
   if (!s) return AMJ_ERR_ARG;
   std::lock_guard<std::mutex> g(s->gpu);
   const uint64_t arena = s->arena_ready ? s->ctx->arena.size : 0;
-  if (resident_bytes)
-    *resident_bytes = s->ctx->allocated > arena ? s->ctx->allocated - arena : 0;
+  const uint64_t held = s->ctx->blocks.held();
+  if (resident_bytes) *resident_bytes = held > arena ? held - arena : 0;
   if (budget_bytes) *budget_bytes = s->budget;
   if (device_free_bytes) {
     size_t f = 0, t = 0;
     if (hipMemGetInfo(&f, &t) != hipSuccess) f = 0;
-    *device_free_bytes = f;
+    *device_free_bytes = f + s->ctx->blocks.parked();  // given back when needed
   }
   return AMJ_OK;
 }

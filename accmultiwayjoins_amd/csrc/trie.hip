@@ -272,10 +272,10 @@ int trie_from_host(amj_ctx_t* ctx, uint64_t n0, const int32_t* d0, const uint64_
 void free_trie(amj_ctx_t* ctx, TrieDev* t) {
   if (!t) return;
   if (ctx) (void)hipStreamSynchronize(ctx->stream);
-  dfree(ctx, t->d0, (uint64_t)t->n0 * 4);
-  dfree(ctx, t->off, ((uint64_t)t->n0 + 1) * 4);
-  dfree(ctx, t->d1, ((uint64_t)t->n1 + kTriePad) * 4);
-  dfree(ctx, t->vrange, (uint64_t)t->vrange_n * 8);
+  dfree(ctx, t->d0);
+  dfree(ctx, t->off);
+  dfree(ctx, t->d1);
+  dfree(ctx, t->vrange);
   *t = TrieDev{};
 }
 

@@ -160,9 +160,10 @@ int amj_sync(amj_ctx_t* ctx);
 /* Pinned host memory (hipHostMalloc) for relations kept on the host (AMJ_REL_HOST): the
  * out-of-core probe streams it to the device at PCIe rate, overlapped with the probe. */
 int amj_host_alloc(size_t bytes, void** out);
-/* Device bytes held by the context now and at its peak (the HBM budget counts the former).
- * Released blocks that the context keeps for its next
- * allocations (at most 2 GiB, given back when an allocation fails) are not counted. */
+/* Device bytes held by the context now and at its peak, as allocated (the HBM budget counts the
+ * former): a request is rounded up to 4 KiB, from 1 to 512 MiB to 64 KiB. Released blocks that the
+ * context keeps for its next allocations (at most 2 GiB) are not counted; they are given back when
+ * an allocation fails. */
 int amj_memory_info(amj_ctx_t* ctx, uint64_t* allocated, uint64_t* peak);
 void amj_host_free(void* p);
 int amj_device_info(amj_ctx_t* ctx, char* name, size_t name_len, uint64_t* hbm_bytes,
@@ -353,7 +354,8 @@ int amj_server_triejoin_runs(amj_server_t* server, uint64_t* runs);
  * reserved again at that size then. */
 int amj_server_set_budget(amj_server_t* server, uint64_t hbm_budget_bytes);
 /* Device bytes held for registered relations and their tables, the result budget, and the
- * device memory free now (any pointer may be NULL). */
+ * device memory free now, released blocks that the context keeps included (any pointer may be
+ * NULL). */
 int amj_server_memory(amj_server_t* server, uint64_t* resident_bytes, uint64_t* budget_bytes,
                       uint64_t* device_free_bytes);
 int amj_server_release(amj_server_t* server, amj_result_t* res);

@@ -8,6 +8,14 @@ from accmultiwayjoins_amd import AmjError
 pytestmark = pytest.mark.gpu
 
 
+def _device_free():
+    """Free bytes of the device, from the HIP runtime that the library has loaded."""
+    import ctypes as C
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
 @pytest.fixture
 def own():
     """A context of its own: its figures are those of the test alone."""
@@ -49,3 +57,40 @@ def test_a_budget_counts_the_tables_whole(own):
     assert r.count == n
     for x in (table, probe, build):
         x.close()
+
+
+def test_memory_info_covers_what_the_device_gave(own):
+    """Blocks of awkward sizes: what the device has less is what the context says it holds, up to
+    2 MiB a block (the granularity of the device's own bookkeeping), and little more than was
+    asked for."""
+    from accmultiwayjoins_amd.serving import DeviceColumns
+    rows = [33_600_001, 33_700_001, 17_000_777, 8_400_003, 300_007, 1_100_003]
+    own.relation([np.zeros(1, np.int32)], [0]).close()
+    free0, held0 = _device_free(), own.allocated_bytes()
+    cols = [DeviceColumns(own, n) for n in rows]
+    taken = free0 - _device_free()
+    held = own.allocated_bytes() - held0
+    asked = sum(2 * 4 * n for n in rows)
+    assert asked <= held <= asked + 2 * len(rows) * (64 << 10)
+    assert taken <= held + 2 * len(rows) * (2 << 20)
+    for c in cols:
+        c.close()
+    assert own.allocated_bytes() == held0
+
+
+def test_a_block_freed_with_another_size_is_not_reused_past_its_end(own):
+    """amj_device_free with more bytes than were allocated: the next allocation of that size gets
+    a block of its own, which holds it."""
+    import ctypes as C
+    from accmultiwayjoins_amd import _native as N
+    from accmultiwayjoins_amd.serving import DeviceColumns
+    held = own.allocated_bytes()
+    p = C.c_void_p()
+    own._check(N.lib().amj_device_alloc(own.h, 1 << 16, C.byref(p)))
+    first = p.value
+    N.lib().amj_device_free(own.h, first, 48 << 20)
+    assert own.allocated_bytes() == held
+    n = (48 << 20) // 4
+    c = DeviceColumns(own, n, ncols=1)
+    assert c.ptrs[0] != first
+    c.close()

@@ -6,7 +6,7 @@
 // for 256 MB, more when the memory has to be cleared first. So a released block of up to kParkBlock
 // bytes is parked, for a later request of its size (the context's work is in stream order, so it is
 // reused without a wait); at most kParkTotal bytes and kParkCount blocks, oldest out first. Parked
-// blocks are given back when an allocation fails.
+// blocks are given back when an allocation fails, in this context or in another one of the device.
 #pragma once
 
 #include <stddef.h>
@@ -32,17 +32,29 @@ constexpr size_t block_bytes(size_t bytes) {
   return bytes > kParkBlock ? bytes : bytes == 0 ? g : (bytes + g - 1) / g * g;
 }
 
-// Device: copyable; int get(size_t bytes, void** p), 0 on success; put(void* p).
+// Device: copyable; operator== (the same device); int get(size_t bytes, void** p), 0 on success;
+// put(void* p); drain(), which waits for all work on the device.
 template <typename Device>
 class Blocks {
  public:
-  explicit Blocks(const Device& dev) : dev_(dev) {}
+  explicit Blocks(const Device& dev) : dev_(dev) {
+    std::lock_guard<std::mutex> g(registry().mu);
+    registry().all.push_back(this);
+  }
   Blocks(const Blocks&) = delete;
   Blocks& operator=(const Blocks&) = delete;
-  ~Blocks() { clear(); }
+  ~Blocks() {
+    {
+      std::lock_guard<std::mutex> g(registry().mu);
+      auto& all = registry().all;
+      all.erase(std::find(all.begin(), all.end(), this));
+    }
+    clear();
+  }
 
   // A block of at least `bytes`. When the device has none, give_way() (what else the context can do
-  // without) and the parked blocks go back to it. 0, or what Device::get returned last.
+  // without), this context's parked blocks and then those of the device's other contexts go back
+  // to it. 0, or what Device::get returned last.
   template <typename GiveWay>
   int take(size_t bytes, void** p, GiveWay&& give_way) {
     const size_t size = block_bytes(bytes);
@@ -64,6 +76,8 @@ class Blocks {
         clear();
         rc = dev_.get(size, p);
       }
+      // other threads may take what was given back, and park again
+      while (rc != 0 && others_give_way()) rc = dev_.get(size, p);
       if (rc != 0) {
         *p = nullptr;
         return rc;
@@ -77,7 +91,7 @@ class Blocks {
   }
 
   // Releases a block: parked if it may be, else given back. Its size is the one it was taken with;
-  // a block of another context goes back to the device.
+  // a block of another context leaves that one's books and goes back to the device.
   void give(void* p, bool park) {
     if (!p) return;
     std::vector<Block> out;
@@ -86,7 +100,7 @@ class Blocks {
       const auto it = sizes_.find(p);
       if (it == sizes_.end()) {
         g.unlock();
-        dev_.put(p);
+        give_foreign(dev_, p);
         return;
       }
       const size_t size = it->second;
@@ -107,6 +121,23 @@ class Blocks {
     for (const Block& b : out) dev_.put(b.first);
   }
 
+  // Releases a block of whichever context holds it, or of one that is gone.
+  static void give_foreign(const Device& dev, void* p) {
+    {
+      std::lock_guard<std::mutex> r(registry().mu);
+      for (Blocks* b : registry().all) {
+        std::lock_guard<std::mutex> g(b->mu_);
+        const auto it = b->sizes_.find(p);
+        if (it == b->sizes_.end()) continue;
+        b->held_ -= it->second;
+        b->sizes_.erase(it);
+        break;
+      }
+    }
+    Device d = dev;
+    d.put(p);
+  }
+
   // Gives all parked blocks back.
   void clear() {
     std::vector<Block> out;
@@ -122,18 +153,45 @@ class Blocks {
     std::lock_guard<std::mutex> g(mu_);
     return peak_;
   }
-  uint64_t parked() const {
-    std::lock_guard<std::mutex> g(mu_);
-    return parked_bytes_;
+  // Bytes parked by all contexts of the device: there for an allocation that needs them.
+  uint64_t parked_on_device() const {
+    std::lock_guard<std::mutex> r(registry().mu);
+    uint64_t n = 0;
+    for (const Blocks* b : registry().all) {
+      if (!(b->dev_ == dev_)) continue;
+      std::lock_guard<std::mutex> g(b->mu_);
+      n += b->parked_bytes_;
+    }
+    return n;
   }
 
  private:
   using Block = std::pair<void*, size_t>;
+  struct Registry {
+    std::mutex mu;  // before any context's own
+    std::vector<Blocks*> all;
+  };
+  static Registry& registry() {
+    static Registry* r = new Registry;  // contexts may end after static objects do
+    return *r;
+  }
+
   void take_parked(std::vector<Block>* out) {
     std::lock_guard<std::mutex> g(mu_);
     out->insert(out->end(), parked_.begin(), parked_.end());
     parked_.clear();
     parked_bytes_ = 0;
+  }
+
+  bool others_give_way() {
+    std::lock_guard<std::mutex> r(registry().mu);
+    std::vector<Block> out;
+    for (Blocks* b : registry().all)
+      if (b != this && b->dev_ == dev_) b->take_parked(&out);
+    if (out.empty()) return false;
+    dev_.drain();  // their contexts' streams may still be at work on them
+    for (const Block& b : out) dev_.put(b.first);
+    return true;
   }
 
   mutable std::mutex mu_;

@@ -36,7 +36,7 @@ int dmalloc(amj_ctx_t* ctx, void** p, size_t bytes) {
 
 void dfree(amj_ctx_t* ctx, void* p) {
   if (ctx) ctx->blocks.give(p, true);
-  else if (p) HipDevice{}.put(p);
+  else if (p) Blocks<HipDevice>::give_foreign(HipDevice{}, p);
 }
 
 int stage_upload(amj_ctx_t* ctx, void* dst, const void* const* src, const size_t* at,
@@ -478,7 +478,7 @@ int finish_checksum(amj_ctx_t* ctx, const uint64_t* block_sums, uint64_t nb, uin
 uint64_t budget_left(amj_ctx_t* ctx, const amj_opts_t* o) {
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-  uint64_t left = free_b + ctx->pool_bytes + ctx->blocks.parked();  // given back when needed
+  uint64_t left = free_b + ctx->pool_bytes + ctx->blocks.parked_on_device();  // given back when needed
   if (ctx->arena.base) left = arena_largest(ctx);
   if (o && o->hbm_budget_bytes) {
     const uint64_t held = ctx->blocks.held();

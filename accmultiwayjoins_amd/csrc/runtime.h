@@ -15,12 +15,14 @@ namespace amj {
 // A context's device, for its Blocks.
 struct HipDevice {
   int id = 0;
+  bool operator==(const HipDevice& o) const { return id == o.id; }
   int get(size_t bytes, void** p) {
     const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) (void)hipGetLastError();
     return (int)e;
   }
   void put(void* p) { (void)hipFree(p); }
+  void drain() { (void)hipDeviceSynchronize(); }
 };
 
 }  // namespace amj

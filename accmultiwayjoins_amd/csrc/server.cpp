@@ -596,7 +596,7 @@ int amj_server_memory(amj_server_t* s, uint64_t* resident_bytes, uint64_t* budge
   if (device_free_bytes) {
     size_t f = 0, t = 0;
     if (hipMemGetInfo(&f, &t) != hipSuccess) f = 0;
-    *device_free_bytes = f + s->ctx->blocks.parked();  // given back when needed
+    *device_free_bytes = f + s->ctx->blocks.parked_on_device();  // given back when needed
   }
   return AMJ_OK;
 }

@@ -163,7 +163,7 @@ int amj_host_alloc(size_t bytes, void** out);
 /* Device bytes held by the context now and at its peak, as allocated (the HBM budget counts the
  * former): a request is rounded up to 4 KiB, from 1 to 512 MiB to 64 KiB. Released blocks that the
  * context keeps for its next allocations (at most 2 GiB) are not counted; they are given back when
- * an allocation fails. */
+ * an allocation fails, in any context of the device in this process. */
 int amj_memory_info(amj_ctx_t* ctx, uint64_t* allocated, uint64_t* peak);
 void amj_host_free(void* p);
 int amj_device_info(amj_ctx_t* ctx, char* name, size_t name_len, uint64_t* hbm_bytes,
@@ -354,7 +354,7 @@ int amj_server_triejoin_runs(amj_server_t* server, uint64_t* runs);
  * reserved again at that size then. */
 int amj_server_set_budget(amj_server_t* server, uint64_t hbm_budget_bytes);
 /* Device bytes held for registered relations and their tables, the result budget, and the
- * device memory free now, released blocks that the context keeps included (any pointer may be
+ * device memory free now, released blocks that contexts keep included (any pointer may be
  * NULL). */
 int amj_server_memory(amj_server_t* server, uint64_t* resident_bytes, uint64_t* budget_bytes,
                       uint64_t* device_free_bytes);

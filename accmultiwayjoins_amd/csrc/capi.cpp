@@ -173,6 +173,12 @@ static size_t owned_col_bytes(uint64_t rows) {
 
 int amj_relation_create(amj_ctx_t* ctx, const amj_rel_t* r, amj_relation_t** out) {
   if (!ctx || !r || !out) return AMJ_ERR_ARG;
+  return create_relation(ctx, r, true, out);
+}
+
+}  // extern "C"
+
+int amj::create_relation(amj_ctx_t* ctx, const amj_rel_t* r, bool wait, amj_relation_t** out) {
   *out = nullptr;
   if (r->num_cols < 1 || r->num_cols > AMJ_MAX_PROBE_COLS || !r->cols) {
     set_error(ctx, AMJ_ERR_ARG, "relations must have 1 or 2 int32 columns");
@@ -210,7 +216,7 @@ int amj_relation_create(amj_ctx_t* ctx, const amj_rel_t* r, amj_relation_t** out
         at[c] = step * c;
         n[c] = bytes;
       }
-      rc = stage_upload(ctx, rel->cols[0], src, at, n, (int)r->num_cols);
+      rc = stage_upload(ctx, rel->cols[0], src, at, n, (int)r->num_cols, wait);
     } else if (bytes > 0) {
       hipError_t e = hipSuccess;
       for (uint32_t c = 0; c < r->num_cols && e == hipSuccess; ++c)
@@ -231,6 +237,8 @@ int amj_relation_create(amj_ctx_t* ctx, const amj_rel_t* r, amj_relation_t** out
   *out = rel.release();
   return AMJ_OK;
 }
+
+extern "C" {
 
 void amj_relation_destroy(amj_ctx_t* ctx, amj_relation_t* rel) {
   if (!rel) return;
@@ -288,7 +296,7 @@ int amj_chain_join(amj_ctx_t* ctx, const amj_rel_t* rels, uint32_t n, const amj_
   std::vector<amj_hash_table_t*> H(n - 1, nullptr);
   int rc = AMJ_OK;
   double build_ms = 0.0;
-  for (uint32_t i = 0; i < n && rc == AMJ_OK; ++i) rc = amj_relation_create(ctx, &rels[i], &R[i]);
+  for (uint32_t i = 0; i < n && rc == AMJ_OK; ++i) rc = create_relation(ctx, &rels[i], false, &R[i]);
   // a build table needs value-sorted runs when its second attribute is bound earlier
   std::vector<uint32_t> seen;
   if (rc == AMJ_OK)
@@ -327,7 +335,7 @@ int amj_pattern_join(amj_ctx_t* ctx, const amj_rel_t* edges, int query, const am
   e.attr_ids = ids01;
   amj_relation_t* R = nullptr;
   amj_hash_table_t* H = nullptr;
-  int rc = amj_relation_create(ctx, &e, &R);
+  int rc = create_relation(ctx, &e, false, &R);
   // one table on the first column, aliased at every level (QueryProcessor.cuh:112-169)
   if (rc == AMJ_OK) rc = amj_hash_table_build(ctx, R, 0, 1, &H);
   if (rc == AMJ_OK) {

@@ -635,7 +635,7 @@ int alftj_trie_build(amj_ctx_t* ctx, const amj_rel_t* rel, amj_trie_t** out) {
     return AMJ_ERR_ARG;
   }
   amj_relation_t* R = nullptr;
-  AMJ_TRY(amj_relation_create(ctx, rel, &R));
+  AMJ_TRY(create_relation(ctx, rel, false, &R));
   const int rc = alftj_trie_build_resident(ctx, R, out);
   amj_relation_destroy(ctx, R);
   return rc;

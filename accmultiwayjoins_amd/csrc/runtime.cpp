@@ -40,7 +40,7 @@ void dfree(amj_ctx_t* ctx, void* p) {
 }
 
 int stage_upload(amj_ctx_t* ctx, void* dst, const void* const* src, const size_t* at,
-                 const size_t* bytes, int n) {
+                 const size_t* bytes, int n, bool wait) {
   const size_t total = (at[n - 1] + bytes[n - 1] + 255) / 256 * 256;
   if (ctx->staging_used + total > kStaging) {  // earlier copies may still be reading it
     AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -51,6 +51,10 @@ int stage_upload(amj_ctx_t* ctx, void* dst, const void* const* src, const size_t
   AMJ_HIP_TRY(ctx, hipMemcpyAsync(dst, p, at[n - 1] + bytes[n - 1], hipMemcpyHostToDevice,
                                   ctx->stream));
   ctx->staging_used += total;
+  if (wait) {
+    AMJ_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->staging_used = 0;
+  }
   return AMJ_OK;
 }
 

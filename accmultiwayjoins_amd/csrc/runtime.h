@@ -122,12 +122,13 @@ enum ScratchSlot {
 // Device memory (blocks.h). ctx may be nullptr for dfree: the block goes back to the device.
 int dmalloc(amj_ctx_t* ctx, void** p, size_t bytes);
 void dfree(amj_ctx_t* ctx, void* p);
-// Columns of up to kStagedCopy bytes are uploaded through the staging buffer: the caller's memory is
-// read before the call returns, the copy is only enqueued. Downloads wait.
+// The columns of a relation of up to kStagedCopy bytes (all columns together) are uploaded through
+// the staging buffer: the caller's memory is read before the call returns, the copy is only enqueued
+// (wait: it is also over). Downloads of up to kStagedCopy bytes pass through it too, and wait.
 constexpr size_t kStaging = 2u << 20;
 constexpr size_t kStagedCopy = 512u << 10;
 int stage_upload(amj_ctx_t* ctx, void* dst, const void* const* src, const size_t* at,
-                 const size_t* bytes, int n);
+                 const size_t* bytes, int n, bool wait);
 int stage_download(amj_ctx_t* ctx, void* dst, const void* src, size_t bytes);
 // Park a result buffer for reuse (at most 256 buffers and a third of the device, oldest
 // out first).
@@ -153,6 +154,10 @@ enum MailWord {
   MAIL_FIB = 16,       // kMaxLevels + 1 words
   MAIL_WORDS = 64
 };
+
+// amj_relation_create; wait = false: small columns may still be on their way, in the order of the
+// context's stream (for relations that no other context sees).
+int create_relation(amj_ctx_t* ctx, const amj_rel_t* r, bool wait, amj_relation_t** out);
 
 // A table as used by one query: the same physical table may be used several times with
 // different attribute ids (the TRI and FOUR queries alias one edge table).

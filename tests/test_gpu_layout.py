@@ -79,3 +79,23 @@ def test_window_written_results_at_ragged_lengths(ctx, n, suffix):
             assert got.checksum == want.checksum
         a, b = (np.stack(r.cols, 1) for r in (got, want))
         assert np.array_equal(a[np.lexsort(a.T)], b[np.lexsort(b.T)])
+
+
+def test_a_relation_is_there_for_another_context_when_the_call_returns(ctx):
+    """Small relations made through one context and read at once by another one's stream."""
+    from accmultiwayjoins_amd import Context
+    with Context(0) as other:
+        for i in range(200):
+            n = 60_001 + i  # two columns below the staging limit
+            rng = np.random.default_rng(i)
+            key = rng.permutation(n).astype(np.int32)
+            val = rng.integers(-2**31, 2**31, n).astype(np.int32)
+            build = ctx.relation([key, val], [1, 2])
+            table = other.hash_table(build)
+            probe = ctx.relation([val, key], [0, 1])
+            r = other.execute(probe, [table], fetch=True)
+            assert r.count == n
+            assert np.array_equal(r.cols[0], val) and np.array_equal(r.cols[2], val)
+            table.close()
+            probe.close()
+            build.close()

@@ -30,7 +30,7 @@ def test_trie_levels_are_the_sorted_distinct_pairs(ctx, n, kind):
     t.close()
 
 
-@pytest.mark.parametrize("n", [1, 1023, 131_071, 131_072, 131_073, 300_001])
+@pytest.mark.parametrize("n", [1, 1023, 65_535, 65_536, 65_537, 131_071, 131_072, 131_073, 300_001])
 def test_uploads_do_not_alias_the_callers_arrays(ctx, n):
     """Columns are the call's: writing over the arrays right after relation() returns, and
     reusing the freed blocks of an earlier relation, leaves what was uploaded. Rows come back
@@ -99,3 +99,22 @@ def test_a_relation_is_there_for_another_context_when_the_call_returns(ctx):
             table.close()
             probe.close()
             build.close()
+
+
+def test_more_columns_in_one_call_than_the_staging_buffer_holds(ctx):
+    """Six relations of just under 512 KB each: the buffer of 2 MB is started over while copies out
+    of it may still be running."""
+    n = 65_000
+    rng = np.random.default_rng(6)
+    rels = [([np.arange(n, dtype=np.int32), rng.permutation(n).astype(np.int32)], [0, 1])]
+    rels += [([np.arange(n, dtype=np.int32), rng.permutation(n).astype(np.int32)], [t, t + 1])
+             for t in range(1, 6)]
+    want = [rels[0][0][0], rels[0][0][1]]
+    for cols, _ids in rels[1:]:
+        want.append(cols[1][want[-1]])
+    for _ in range(3):
+        r = ctx.chain_join(rels, fetch=True)
+        assert r.count == n
+        order = np.argsort(r.cols[0], kind="stable")
+        for got, w in zip(r.cols, want):
+            assert np.array_equal(got[order], w)

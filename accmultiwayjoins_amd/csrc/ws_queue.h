@@ -22,10 +22,10 @@ namespace amj {
 
 // Control block of one launch (zeroed by the host). Updates of one cache line serialise across
 // the device (tens of ns each), so what is updated often has a line of its own, and units are
-// claimed from kUnitShards counters (unit u belongs to shard u % kUnitShards; a wave starts with
-// the shard of its workgroup's XCD and goes on to the others). Count of a 1 M-row chain (15,625
+// claimed from kUnitShards counters (ws_split.h; a wave starts with the shard of its workgroup's
+// XCD and goes on to the others). Count of a 1 M-row chain (15,625
 // units): 1.25 ms with one counter, 0.85 with eight.
-constexpr uint32_t kUnitShards = kXcds;
+static_assert(kUnitShards == kXcds, "one claim counter per XCD");
 struct alignas(128) WsShard {
   unsigned long long next;  // units of the shard claimed
 };
@@ -43,8 +43,6 @@ struct alignas(128) WsCtl {
   unsigned long long pushed;     // tasks published
 };
 
-constexpr uint64_t kMaxClaim = 64;  // units claimed at once by a wave
-constexpr uint64_t kMinClaim = 4;   // ... and at least, in launches of many units per wave
 constexpr uint32_t kFlagSpin = 1u;
 // Frontier steps of 64 children between two progress reports of a working wave: idle waves
 // then see progress while a wave walks a long level alone, not only when a unit or a task ends.
@@ -174,27 +172,19 @@ __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
     working = on;
   };
   for (;;) {
-    // Guided chunks of at most 64 units. With 16 or more units per wave: half the remaining ones
-    // per wave and at least 4, so that cheap units do not pay for a claim each. With fewer (the
-    // triejoin's units of many roots, heaviest first): a quarter and at least 1; 4 units at a time
-    // took the 4-cliques of R-MAT 20 from 290 to 860 ms.
     if (units_left) {
       uint64_t u = 0, n = 0;
       uint32_t tried = 0;
       for (; tried < kUnitShards; ++tried) {
-        const uint64_t size = (A.units + kUnitShards - 1 - shard) / kUnitShards;
+        const uint64_t size = ws_shard_units(A.units, shard);
         if (lane_id() == 0) {
           unsigned long long* next = &A.ctl->shard[shard].next;
           const unsigned long long at = ld_rlx(next);
           if (at < size) {
-            const uint64_t waves = (uint64_t)gridDim.x * kWavesPerBlock;
-            const uint64_t most = A.max_claim ? A.max_claim : kMaxClaim;
-            const bool many = A.units >= 16 * waves;
-            const uint64_t least = (many && most >= kMinClaim) ? kMinClaim : 1;
-            uint64_t k = (size - at) * kUnitShards / ((many ? 2 : 4) * waves);
-            k = k < least ? least : (k > most ? most : k);
+            const uint64_t k = ws_claim(A.units, size, at, (uint64_t)gridDim.x * kWavesPerBlock,
+                                        A.max_claim);
             u = add_relaxed(next, (unsigned long long)k);
-            n = u < size ? (k < size - u ? k : size - u) : 0;
+            n = ws_granted(u, k, size);
           }
         }
         n = lane0_u64(n);
@@ -203,7 +193,7 @@ __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
       }
       if (n) {
         work(true);
-        const uint64_t first = lane0_u64(u) * kUnitShards + shard;
+        const uint64_t first = ws_unit_of_shard(lane0_u64(u), shard);
         run_units(first, first + n * kUnitShards, kUnitShards);
         continue;
       }
@@ -235,8 +225,8 @@ __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
         __hip_atomic_fetch_or(&A.ctl->flags, kFlagSpin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       break;
     }
-    // idle waves look again after 2, 4, .. 14 us, so that thousands of them leave the counters to
-    // the waves that work
+    // idle waves look again after one, two, four and then eight naps of 64 x 64 cycles (about 2 us
+    // each), so that thousands of them leave the counters to the waves that work
     for (int i = 0; i < naps; ++i) __builtin_amdgcn_s_sleep(64);
     naps = naps < 8 ? 2 * naps : 8;
   }

@@ -1,12 +1,14 @@
 // CPU model of the work-sharing protocol of the persistent engines (ws_queue.h), restated with
-// C++ atomics on many host threads, plus an exhaustive check of the range arithmetic both GPU
+// C++ atomics on many host threads, plus a check of the range and claim arithmetic both GPU
 // engines share (ws_split.h, compiled here unchanged).
 //
 // The reference's substrate (TaskBook.cuh:13-109 task append, GCQueue.cuh:30-107 tagged CAS
 // queue, CBarrier.cuh:9-46 idle barrier) has no capacity check; the protocol modelled here
-// reserves slots with a clamped fetch-add, publishes each record with a release store of its
-// own flag, claims with a CAS on the head, and ends when no unit is left, no published task is
-// unclaimed and nobody holds work, with every wait bounded.
+// claims units from several counters (every worker starts at its own and goes on to the others),
+// reserves task slots with a clamped fetch-add, publishes each record with a release store of its
+// own flag, claims it with a CAS on the head, and ends when no unit is left, no published task is
+// unclaimed and nobody holds work, with every wait bounded. A worker counts as busy from its first
+// claim until it finds no work.
 //
 // A "unit" u owns W(u) children (heavily skewed); a worker walks a range 64 children at a
 // time and, when more than split + 64 are left, shares the tail as tasks, exactly as
@@ -86,9 +88,52 @@ static void check_split_math() {
   std::printf("split arithmetic: %llu cases ok\n", (unsigned long long)cases);
 }
 
-// ---- 2. the protocol ------------------------------------------------------------------------
+// ---- 2. claim arithmetic ----------------------------------------------------------------
+// Shards and claims give every unit once, whatever the number of units, waves and the cap.
+static void check_claim_math() {
+  uint64_t cases = 0;
+  for (uint64_t units = 0; units <= 5 * kUnitShards + 1; ++units) {
+    uint64_t sum = 0;
+    std::vector<int> seen(units, 0);
+    for (uint32_t s = 0; s < kUnitShards; ++s) {
+      const uint64_t size = ws_shard_units(units, s);
+      sum += size;
+      for (uint64_t k = 0; k < size; ++k) {
+        const uint64_t u = ws_unit_of_shard(k, s);
+        CHECK(u < units && u % kUnitShards == s, "unit %llu of shard %u", (unsigned long long)u, s);
+        ++seen[u];
+      }
+    }
+    CHECK(sum == units, "shards hold %llu of %llu units", (unsigned long long)sum,
+          (unsigned long long)units);
+    for (int n : seen) CHECK(n == 1, "a unit in %d shards", n);
+  }
+  for (uint64_t units : {1ull, 7ull, 9ull, 63ull, 64ull, 100ull, 255ull, 256ull, 5000ull, 312500ull})
+    for (uint64_t waves : {1ull, 4ull, 16ull, 4096ull})
+      for (uint64_t cap : {0ull, 1ull, 2ull, 3ull, 64ull})
+        for (uint32_t s = 0; s < kUnitShards; ++s) {
+          const uint64_t size = ws_shard_units(units, s);
+          uint64_t at = 0, got = 0;  // one worker after the other, as the counter orders them
+          while (at < size) {
+            const uint64_t k = ws_claim(units, size, at, waves, cap);
+            CHECK(k >= 1 && k <= (cap ? cap : kMaxClaim), "claim of %llu", (unsigned long long)k);
+            CHECK(units < kManyUnits * waves || (cap && cap < kMinClaim) || k >= kMinClaim,
+                  "claim of %llu with many units per wave", (unsigned long long)k);
+            got += ws_granted(at, k, size);
+            at += k;
+            ++cases;
+          }
+          CHECK(got == size, "claims gave %llu of %llu units", (unsigned long long)got,
+                (unsigned long long)size);
+          CHECK(ws_granted(at, 5, size) == 0, "granted past the shard");
+        }
+  std::printf("claim arithmetic: %llu claims ok\n", (unsigned long long)cases);
+}
+
+// ---- 3. the protocol ------------------------------------------------------------------------
 struct Ctl {
-  std::atomic<uint64_t> next_unit{0}, q_tail{0}, q_head{0}, pushed{0}, progress{0};
+  std::atomic<uint64_t> shard[kUnitShards] = {};
+  std::atomic<uint64_t> q_tail{0}, q_head{0}, pushed{0}, progress{0};
   std::atomic<uint32_t> busy{0}, flags{0};
 };
 
@@ -98,12 +143,13 @@ struct Task {
 
 struct Model {
   uint64_t units, split, cap, stall_ns;
-  uint64_t max_claim = 64;  // WsArgs::max_claim (kMaxClaim when 0 there)
+  uint64_t max_claim = 0;  // WsArgs::max_claim
   int workers;
   bool withhold_one;  // a worker reserves a slot and never publishes it (the stuck case)
   std::vector<uint64_t> width;          // children per unit
   std::vector<uint64_t> first;          // offset of a unit's children in `visits`
   std::vector<std::atomic<uint32_t>> visits;
+  std::vector<std::atomic<uint32_t>> unit_runs;
   std::vector<Task> tasks;
   std::vector<std::atomic<uint32_t>> ready;
   Ctl ctl;
@@ -122,6 +168,7 @@ struct Model {
     }
     first[u] = total;
     visits = std::vector<std::atomic<uint32_t>>(total);
+    unit_runs = std::vector<std::atomic<uint32_t>>(u);
   }
 
   static uint64_t now_ns() {
@@ -143,8 +190,12 @@ struct Model {
   }
 
   // ws_ldescend over one unit's children [c0, c1)
-  void walk(uint64_t unit, uint64_t c0, uint64_t c1, bool& qfull) {
+  struct Worker {
+    bool qfull = false;
+  };
+  void walk(uint64_t unit, uint64_t c0, uint64_t c1, Worker& w) {
     uint64_t end = c1;
+    bool& qfull = w.qfull;
     for (uint64_t c = c0; c < end; c += 64) {
       if (!qfull && ws_should_split(c, end, split)) {
         const uint64_t k = ws_pieces(c, end, split);
@@ -189,45 +240,53 @@ struct Model {
     return -1;
   }
 
-  // ws_serve
-  void serve() {
-    bool qfull = false;
+  // ws_serve of worker number id
+  void serve(int id) {
+    Worker w;
     uint64_t seen = ~0ull, since = 0;
+    bool units_left = true, working = false;
+    uint32_t shard = (uint32_t)id % kUnitShards;
+    const auto work = [&](bool on) {
+      if (split && on != working) ctl.busy.fetch_add(on ? 1u : ~0u, std::memory_order_relaxed);
+      working = on;
+    };
     for (;;) {
-      uint64_t u = ~0ull, nu = 0;
-      const uint64_t seen_u = ctl.next_unit.load(std::memory_order_relaxed);
-      if (seen_u < units) {
-        // guided claims: half the remaining units per worker and at least 4 with 64 or more
-        // units per worker, else a quarter and at least 1; at most max_claim
-        const bool many = units >= 64 * (uint64_t)workers;
-        const uint64_t least = (many && max_claim >= 4) ? 4 : 1;
-        uint64_t k = (units - seen_u) / ((many ? 2 : 4) * (uint64_t)workers);
-        k = k < least ? least : (k > max_claim ? max_claim : k);
-        u = ctl.next_unit.fetch_add(k, std::memory_order_relaxed);
-        nu = k;
-      }
-      if (u < units) {
-        const uint64_t ue = std::min(u + nu, units);
-        // busy and progress serve only the waits for tasks
-        if (split) ctl.busy.fetch_add(1, std::memory_order_relaxed);
-        for (uint64_t v = u; v < ue; ++v) walk(v, 0, width[v], qfull);
-        if (split) {
-          ctl.progress.fetch_add(1, std::memory_order_relaxed);
-          ctl.busy.fetch_sub(1, std::memory_order_relaxed);
+      if (units_left) {
+        uint64_t u = 0, n = 0;
+        for (uint32_t tried = 0; tried < kUnitShards; ++tried) {
+          const uint64_t size = ws_shard_units(units, shard);
+          const uint64_t at = ctl.shard[shard].load(std::memory_order_relaxed);
+          if (at < size) {
+            const uint64_t k = ws_claim(units, size, at, (uint64_t)workers, max_claim);
+            u = ctl.shard[shard].fetch_add(k, std::memory_order_relaxed);
+            n = ws_granted(u, k, size);
+          }
+          if (n) break;
+          shard = (shard + 1) % kUnitShards;
         }
-        continue;
+        if (n) {
+          work(true);
+          for (uint64_t k = u; k < u + n; ++k) {
+            const uint64_t v = ws_unit_of_shard(k, shard);
+            CHECK(v < units, "unit %llu of %llu", (unsigned long long)v, (unsigned long long)units);
+            unit_runs[v].fetch_add(1, std::memory_order_relaxed);
+            walk(v, 0, width[v], w);
+          }
+          continue;
+        }
+        units_left = false;
       }
       if (split == 0) break;
       const int64_t slot = try_pop();
       if (slot >= 0) {
-        ctl.busy.fetch_add(1, std::memory_order_relaxed);
+        work(true);
         const Task t = tasks[(uint64_t)slot];
         CHECK(t.unit < units && t.c0 < t.c1 && t.c1 <= width[t.unit], "bad task record");
-        walk(t.unit, t.c0, t.c1, qfull);
+        walk(t.unit, t.c0, t.c1, w);
         ctl.progress.fetch_add(1, std::memory_order_relaxed);
-        ctl.busy.fetch_sub(1, std::memory_order_relaxed);
         continue;
       }
+      work(false);
       if (slot == -2) break;
       if (ctl.busy.load(std::memory_order_relaxed) == 0 &&
           ctl.q_head.load(std::memory_order_relaxed) >= queue_end())
@@ -243,19 +302,20 @@ struct Model {
       }
       std::this_thread::yield();
     }
+    CHECK(!working || split == 0, "a worker left while it counted as busy");
   }
 
   // runs the workers; returns the error flag; every worker must have left
   uint32_t run() {
     std::vector<std::thread> th;
-    for (int w = 0; w < workers; ++w) th.emplace_back([this] { serve(); });
+    for (int w = 0; w < workers; ++w) th.emplace_back([this, w] { serve(w); });
     for (auto& t : th) t.join();
     return ctl.flags.load();
   }
 };
 
 static void run_case(uint64_t units, uint64_t split, uint64_t cap, int workers, uint64_t seed,
-                     uint64_t max_claim = 64) {
+                     uint64_t max_claim = 0) {
   Model m(units, split, cap, workers, seed, false);
   m.max_claim = max_claim;
   const uint32_t flags = m.run();
@@ -264,6 +324,10 @@ static void run_case(uint64_t units, uint64_t split, uint64_t cap, int workers, 
   for (size_t i = 0; i < m.visits.size(); ++i)
     CHECK(m.visits[i].load() == 1, "child %zu visited %u times (split %llu cap %llu)", i,
           m.visits[i].load(), (unsigned long long)split, (unsigned long long)cap);
+  for (uint64_t u = 0; u < units; ++u)
+    CHECK(m.unit_runs[u].load() == 1, "unit %llu claimed %u times", (unsigned long long)u,
+          m.unit_runs[u].load());
+  CHECK(m.ctl.busy.load() == 0, "busy ended at %u", m.ctl.busy.load());
   CHECK(m.ctl.q_head.load() == std::min<uint64_t>(m.ctl.q_tail.load(), cap) || split == 0,
         "published tasks left unclaimed");
   std::printf("units %llu split %llu cap %llu workers %d: %zu children once each, %llu tasks\n",
@@ -273,6 +337,7 @@ static void run_case(uint64_t units, uint64_t split, uint64_t cap, int workers, 
 
 int main() {
   check_split_math();
+  check_claim_math();
   const int hw = (int)std::max(2u, std::min(16u, std::thread::hardware_concurrency()));
   run_case(2000, 0, 16, hw, 1);        // no sharing
   run_case(2000, 1024, 8192, hw, 2);   // the ALFTJ default
@@ -281,10 +346,14 @@ int main() {
   run_case(3000, 256, 1, 3, 5);        // one slot
   run_case(500, 64, 4096, 1, 6);       // one worker serves its own tasks
   run_case(4000, 192, 100000, 64, 7);  // many more workers than cores
-  run_case(12000, 0, 16, hw, 9);       // 64 or more units per worker: claims of at least 4
+  run_case(12000, 0, 16, hw, 9);        // many units per worker: claims of at least 4
   run_case(12000, 1024, 8192, hw, 10);  // ... with sharing
-  run_case(12000, 0, 16, hw, 11, 2);   // claims capped below the minimum of 4
+  run_case(12000, 0, 16, hw, 11, 2);    // claims capped below the minimum of 4
   run_case(12000, 256, 8192, hw, 12, 1);  // single-unit claims with sharing
+  for (uint64_t u : {0, 1, 7, 8, 9, 25}) {  // few units: fewer than shards, than workers
+    run_case(u, 0, 16, hw, 20 + u);
+    run_case(u, 128, 64, hw, 60 + u);
+  }
   // a reserved slot whose flag never comes: the taker gives up with the error flag
   Model m(200, 64, 4096, hw, 8, true);
   m.stall_ns = 200'000'000ull;

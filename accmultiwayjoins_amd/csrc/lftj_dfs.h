@@ -265,6 +265,11 @@ __device__ __forceinline__ bool lchild(const LPlan& P, const LLv<A>& par, uint32
 // whole wave, which keeps the values of one list in LDS and checks the other list's values
 // against them; the rest go through the flattened enumeration.
 constexpr uint32_t kCoopMinCands = 32;
+// What a level reports as it goes: steps of 64 candidates or list values. The unit engine has no use
+// for it; the work-sharing engine's idle waves take it as progress (ws_queue.h).
+struct NoSteps {
+  __device__ __forceinline__ void operator()(uint32_t) const {}
+};
 constexpr uint32_t kStageInts = 1024;  // values of the checked list, at most
 // 4-clique pairs (descend_clique_pairs): the checked list of an entry, and the entry's
 // intersection.
@@ -526,9 +531,9 @@ struct PairLists {
 // lanes that passed. R-MAT 22, count / write with checksum: 31.8 / 43.9 ms before, 27.6 / 35 ms now
 // (880 M lines of 128 B fetched past the L2 per pass, 4.2 TB/s); R-MAT 20, count with checksum 5.6
 // -> 4.6 ms.
-template <int A, uint64_t SH, typename Sink>
+template <int A, uint64_t SH, typename Sink, typename Steps>
 __device__ __forceinline__ void descend_tri_last(const LPlan& P, const LLv<A>& par, Sink& sink,
-                                                 lds_i32* stage) {
+                                                 lds_i32* stage, const Steps& steps) {
   static_assert(A == 3 && SH == kShapeTri, "triangle shape only");
   const uint32_t na = par.hi[1] - par.lo[1], nb = par.hi[2] - par.lo[2];
   const bool coop = par.dlen >= kCoopMinCands && (par.drel == 1 ? nb : na) <= kStageInts;
@@ -538,6 +543,7 @@ __device__ __forceinline__ void descend_tri_last(const LPlan& P, const LLv<A>& p
     finish(sm);
     for (uint32_t c = 0; c < sm.T; c += (uint32_t)kWave) {
       LLv<A> ch;
+      steps(1u);
       const bool ok = lchild<A, 2, SH>(P, sm, c, sm.T, ch);
       sink(ok, ch.b);
     }
@@ -564,6 +570,7 @@ __device__ __forceinline__ void descend_tri_last(const LPlan& P, const LLv<A>& p
       [&](int p) {
         const uint64_t src = readlane_u64((uint64_t)pl.set, p);
         const uint32_t n = readlane_u32(pl.set_n, p);
+        steps(1u + readlane_u32(pl.str_n, p) / kWave);
         if (src == kept && n == set.n) return;
         kept = src;
         set.fill(n, kTriTable, [&](uint32_t i) { return ld_at<true>((const int32_t*)src, i); });
@@ -588,9 +595,9 @@ __device__ __forceinline__ void descend_tri_last(const LPlan& P, const LLv<A>& p
 // lists are copied to the wave's LDS stage once, and each chunk of 64 candidates is checked
 // there by binary searches of uniform length (one global load per candidate instead of a
 // chain of dependent ones). The other entries go through the flattened enumeration.
-template <int A, int I, uint64_t SH, typename Sink>
+template <int A, int I, uint64_t SH, typename Sink, typename Steps>
 __device__ __forceinline__ void descend_last_fixed(const LPlan& P, const LLv<A>& par, Sink& sink,
-                                                   lds_i32* stage) {
+                                                   lds_i32* stage, const Steps& steps) {
   constexpr uint32_t cm = (uint32_t)(SH >> (12 * I + 6)) & 63u;
   constexpr int nc = bit_count(cm);
   static_assert(nc >= 2, "the last attribute has a driver and at least one list to check");
@@ -622,6 +629,7 @@ __device__ __forceinline__ void descend_last_fixed(const LPlan& P, const LLv<A>&
     finish(sm);
     for (uint32_t c = 0; c < sm.T; c += (uint32_t)kWave) {
       LLv<A> ch;
+      steps(1u);
       const bool ok = lchild<A, I, SH>(P, sm, c, sm.T, ch);
       sink(ok, ch.b);
     }
@@ -643,6 +651,7 @@ __device__ __forceinline__ void descend_last_fixed(const LPlan& P, const LLv<A>&
     m &= m - 1;
     const int32_t* dp = (const int32_t*)readlane_u64((uint64_t)par.dptr, p);
     const uint32_t dl = readlane_u32(par.dlen, p);
+    steps(1u + dl / kWave);
     const int32_t* src[no];
     uint32_t n[no];
     bool same = true;
@@ -709,9 +718,9 @@ __device__ __forceinline__ void descend_last_fixed(const LPlan& P, const LLv<A>&
 // fit a CU; one of a quarter of the size, with a fourth workgroup per CU, was slower (R-MAT 18 dense
 // cores have longer L: 72 ms against 44). Searching L instead, chunks flattened over the wave:
 // R-MAT 18 / 20 62 / 298 ms (unit engine, count + checksum), now 44 / 174 ms.
-template <int A, uint64_t SH, typename Sink>
-__device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A>& par,
-                                                     Sink& sink, lds_i32* stage) {
+template <int A, uint64_t SH, typename Sink, typename Steps>
+__device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A>& par, Sink& sink,
+                                                     lds_i32* stage, const Steps& steps) {
   static_assert(A == 4 && SH == kShapeFour, "4-clique shape only");
   constexpr int K = kCoopChunks;
   const uint32_t na = par.hi[1] - par.lo[1], nb = par.hi[3] - par.lo[3];
@@ -724,10 +733,11 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
     finish(sm);
     for (uint32_t c = 0; c < sm.T; c += (uint32_t)kWave) {
       LLv<A> ch;
+      steps(1u);
       const bool ok = lchild<A, 2, SH>(P, sm, c, sm.T, ch);
       choose_driver<A, SH>(P, 3, ok, ch);
       finish(ch);
-      if (ch.T) descend_last_fixed<A, 3, SH>(P, ch, sink, stage);
+      if (ch.T) descend_last_fixed<A, 3, SH>(P, ch, sink, stage, steps);
     }
   }
 
@@ -747,6 +757,7 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
     m &= m - 1;
     const uint64_t src = readlane_u64((uint64_t)pl.set, p);
     const uint32_t n = readlane_u32(pl.set_n, p);
+    steps(1u + readlane_u32(pl.str_n, p) / kWave);
     if (src != kept || n != set.n) {
       kept = src;
       set.fill(n, kFourTable, [&](uint32_t i) { return ld_at<true>((const int32_t*)src, i); });
@@ -787,6 +798,7 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
       const uint32_t clen = f ? chi - clo : 0u;
       const uint32_t incl = wave_scan_add_dpp(clen);
       const uint32_t T = lane63(incl);
+      steps(1u + T / kWave);
       const uint64_t fm = __ballot(f);
       const auto emit = [&]() {
         hits.take([&](bool ok, int32_t v, int q) {
@@ -834,39 +846,41 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
   }
 }
 
-template <int A, int i, uint64_t SH = 0, typename Sink>
+template <int A, int i, uint64_t SH = 0, typename Sink, typename Steps = NoSteps>
 __device__ __forceinline__ void descend(const LPlan& P, const LLv<A>& par, Sink& sink,
-                                        lds_i32* stage = nullptr) {
+                                        lds_i32* stage = nullptr, const Steps& steps = {}) {
   if constexpr (SH == kShapeTri && i == A - 1) {
-    descend_tri_last<A, SH>(P, par, sink, stage);
+    descend_tri_last<A, SH>(P, par, sink, stage, steps);
   } else if constexpr (SH != 0 && i == A - 1) {
-    descend_last_fixed<A, i, SH>(P, par, sink, stage);
+    descend_last_fixed<A, i, SH>(P, par, sink, stage, steps);
   } else if constexpr (SH == kShapeFour && i == 2) {
     // (0,2) and (0,3) one trie, (1,2) and (1,3) another: the clique pairs apply
     const bool same = P.rel[1].d1 == P.rel[2].d1 && P.rel[1].off == P.rel[2].off &&
                       P.rel[1].d0 == P.rel[2].d0 && P.rel[3].d1 == P.rel[4].d1 &&
                       P.rel[3].off == P.rel[4].off && P.rel[3].d0 == P.rel[4].d0;
     if (same) {
-      descend_clique_pairs<A, SH>(P, par, sink, stage);
+      descend_clique_pairs<A, SH>(P, par, sink, stage, steps);
       return;
     }
     for (uint32_t c = 0; c < par.T; c += (uint32_t)kWave) {
       LLv<A> ch;
+      steps(1u);
       const bool ok = lchild<A, i, SH>(P, par, c, par.T, ch);
       choose_driver<A, SH>(P, i + 1, ok, ch);
       finish(ch);
-      if (ch.T) descend<A, i + 1, SH>(P, ch, sink, stage);
+      if (ch.T) descend<A, i + 1, SH>(P, ch, sink, stage, steps);
     }
   } else {
     for (uint32_t c = 0; c < par.T; c += (uint32_t)kWave) {
       LLv<A> ch;
+      steps(1u);
       const bool ok = lchild<A, i, SH>(P, par, c, par.T, ch);
       if constexpr (i == A - 1) {
         sink(ok, ch.b);
       } else {
         choose_driver<A, SH>(P, i + 1, ok, ch);
         finish(ch);
-        if (ch.T) descend<A, i + 1, SH>(P, ch, sink, stage);
+        if (ch.T) descend<A, i + 1, SH>(P, ch, sink, stage, steps);
       }
     }
   }

@@ -106,10 +106,10 @@ __device__ __forceinline__ void ws_ldescend(const LPlan& P, const LLv<A>& par, u
                                             uint32_t c1, Sink& sink, const WsArgs& W,
                                             WsWave& q, lds_i32* stage) {
   if constexpr (coop_level<A, i, SH>()) {
-    ws_step(W, q);
     LLv<A> r = par;
     restrict_range(r, c0, c1);
-    if (r.T) descend<A, i, SH>(P, r, sink, stage);
+    if (r.T)
+      descend<A, i, SH>(P, r, sink, stage, [&](uint32_t n) { ws_step(W, q, n); });
     return;
   }
   uint64_t end = c1;

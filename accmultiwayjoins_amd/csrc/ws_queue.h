@@ -44,9 +44,6 @@ struct alignas(128) WsCtl {
 };
 
 constexpr uint32_t kFlagSpin = 1u;
-// Frontier steps of 64 children between two progress reports of a working wave: idle waves
-// then see progress while a wave walks a long level alone, not only when a unit or a task ends.
-constexpr uint32_t kBeatSteps = 4096;
 
 struct WsArgs {
   WsCtl* ctl;
@@ -87,12 +84,12 @@ __device__ __forceinline__ uint64_t lane0_u64(uint64_t v) {
   return uniform(__shfl(v, 0, kWave));
 }
 
-// One frontier step of a working wave; every kBeatSteps steps it reports progress. A launch
-// without a control block (the size samples) only counts.
-__device__ __forceinline__ void ws_step(const WsArgs& A, WsWave& W) {
-  W.iters += 1u;
-  if (A.ctl && (W.iters % kBeatSteps) == 0u && lane_id() == 0)
-    add_relaxed(&A.ctl->progress, 1ull);
+// n (uniform) steps of a working wave; every kBeatSteps steps it reports progress. A launch without
+// a control block (the size samples) only counts.
+__device__ __forceinline__ void ws_step(const WsArgs& A, WsWave& W, uint32_t n = 1u) {
+  const bool beat = ws_beat(W.iters, n);
+  W.iters += n;
+  if (beat && A.ctl && lane_id() == 0) add_relaxed(&A.ctl->progress, 1ull);
 }
 
 // Reserve up to k task slots with one fetch-add; returns the first slot, the number granted in
@@ -156,10 +153,11 @@ __device__ __forceinline__ int64_t try_pop(const WsArgs& A) {
 // (run_units(first, end, step)), then take tasks (run_task(slot)) until the launch has drained.
 //
 // A claim is one update of one counter. A wave counts as busy from its first claim until it finds
-// no work, not per claim, and reports progress from its heartbeat (ws_step) and per task: with a
-// busy, a progress and a claim update per claim, quarter-size claims down to one unit, and all
-// three counters in one line, counting 20 M probe rows (312,500 units, fan-out 1) took 9.9 ms, of
-// which the lookups are 1.2; now 2.2.
+// no work, not per claim, and reports progress from its heartbeat (ws_step) and per task, not per
+// claim; running out of work is seen in busy (one more update per wave cost 0.25 ms of the 2.5 that
+// counting 20 M probe rows takes). With a busy, a progress and a claim update per claim,
+// quarter-size claims down to one unit, and all three counters in one line, that count (312,500
+// units, fan-out 1) took 9.9 ms, of which the lookups are 1.2.
 template <typename RunUnits, typename RunTask>
 __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
                                          RunTask&& run_task) {
@@ -215,7 +213,9 @@ __device__ __forceinline__ void ws_serve(const WsArgs& A, RunUnits&& run_units,
       done = (ld_rlx(&A.ctl->busy) == 0u && ld_rlx(&A.ctl->q_head) >= queue_end(A)) ? 1u : 0u;
     if (uniform(__shfl(done, 0, kWave))) break;
     // no work here while other waves hold some: give up only if nothing moves for long
-    const uint64_t prog = lane0_u64(lane_id() == 0 ? ld_rlx(&A.ctl->progress) : 0ull);
+    // (a wave that runs out of work moves busy)
+    const uint64_t prog = lane0_u64(
+        lane_id() == 0 ? ws_moved(ld_rlx(&A.ctl->progress), ld_rlx(&A.ctl->busy)) : 0ull);
     const uint64_t now = wall_clock64();
     if (prog != seen) {
       seen = prog;

@@ -63,6 +63,23 @@ constexpr uint64_t ws_claim(uint64_t units, uint64_t size, uint64_t at, uint64_t
   return k < least ? least : (k > most ? most : k);
 }
 
+// Steps of 64 children (or values of a streamed list) between two progress reports of a working
+// wave: idle waves then see progress while others walk long levels, whatever their units and tasks
+// take. A wave's steps count over all its units, and between two of them lie a few loads: reports
+// are 1 to 20 ms apart.
+constexpr uint32_t kBeatSteps = 4096;
+
+// Does a wave that has taken `before` steps report after n more?
+constexpr bool ws_beat(uint32_t before, uint32_t n) {
+  return (before + n) / kBeatSteps != before / kBeatSteps;
+}
+
+// What a waiting wave watches: it changes whenever a wave reports progress, starts to work or runs
+// out of work.
+constexpr uint64_t ws_moved(uint64_t progress, uint32_t busy) {
+  return progress + ((uint64_t)busy << 40);
+}
+
 // Slots granted by one fetch-add on a counter: tail was the old value, cap the capacity (the task
 // queue's, or the units of a shard).
 constexpr uint64_t ws_granted(uint64_t tail, uint64_t want, uint64_t cap) {

@@ -1,6 +1,8 @@
 """Intersections of the compiled triangle and 4-clique shapes at the list lengths and values where
 their variants meet: LDS tables (up to 7/16 of 64 .. 2,048 slots), lists that do not fit or do not
 settle in a table, lists past the stage, streamed and flattened children, duplicates in CSR tries."""
+import math
+
 import numpy as np
 import pytest
 
@@ -105,3 +107,18 @@ def test_cliques_of_complete_graphs(ctx, n, ws):
         w = ctx.lftj_pattern(s, d, "FOUR", "DFS", materialize=True, ws=ws)
         assert (w.count, w.checksum) == (t4.count, t4.checksum)
         ctx.free(w)
+
+
+@pytest.mark.parametrize("query,n,stall", [("FOUR", 512, 50), ("TRI", 1000, 10)])
+def test_ws_long_units_with_progress_are_not_a_stall(ctx, query, n, stall):
+    """K_n in a few units of 64 roots and no tasks (a split longer than any run): a few waves work
+    for much longer than the stall limit while all others are idle. What the working waves
+    report from inside their lists keeps the pass alive."""
+    i, j = np.triu_indices(n, 1)
+    s, d = i.astype(np.int32), j.astype(np.int32)
+    want = ctx.lftj_pattern(s, d, query, "DFS", materialize=False)
+    assert want.count == (math.comb(n, 4) if query == "FOUR" else math.comb(n, 3))
+    r = ctx.lftj_pattern(s, d, query, "DFS", materialize=False, ws=1,
+                         ws_split_threshold=1 << 20, ws_stall_ms=stall)
+    assert (r.count, r.checksum) == (want.count, want.checksum)
+    assert r.detail == 0  # no tasks

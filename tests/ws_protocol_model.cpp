@@ -8,7 +8,8 @@
 // reserves task slots with a clamped fetch-add, publishes each record with a release store of its
 // own flag, claims it with a CAS on the head, and ends when no unit is left, no published task is
 // unclaimed and nobody holds work, with every wait bounded. A worker counts as busy from its first
-// claim until it finds no work.
+// claim until it finds no work; progress is reported from its steps and per task, and a waiting
+// worker also sees others start and run out of work.
 //
 // A "unit" u owns W(u) children (heavily skewed); a worker walks a range 64 children at a
 // time and, when more than split + 64 are left, shares the tail as tasks, exactly as
@@ -127,6 +128,15 @@ static void check_claim_math() {
                 (unsigned long long)size);
           CHECK(ws_granted(at, 5, size) == 0, "granted past the shard");
         }
+  // reports: one per kBeatSteps steps, however the steps come
+  uint32_t steps = 0, beats = 0;
+  for (uint32_t i = 0; steps < 100 * kBeatSteps; ++i) {
+    const uint32_t n = i % 97 + 1;
+    beats += ws_beat(steps, n) ? 1 : 0;
+    steps += n;
+  }
+  CHECK(beats == steps / kBeatSteps, "%u reports in %u steps", beats, steps);
+  CHECK(ws_beat(kBeatSteps - 1, 1) && !ws_beat(kBeatSteps, kBeatSteps - 1), "report early or late");
   std::printf("claim arithmetic: %llu claims ok\n", (unsigned long long)cases);
 }
 
@@ -146,6 +156,8 @@ struct Model {
   uint64_t max_claim = 0;  // WsArgs::max_claim
   int workers;
   bool withhold_one;  // a worker reserves a slot and never publishes it (the stuck case)
+  uint32_t step_weight = 1;  // steps counted for 64 children
+  uint64_t step_us = 0;      // time they take
   std::vector<uint64_t> width;          // children per unit
   std::vector<uint64_t> first;          // offset of a unit's children in `visits`
   std::vector<std::atomic<uint32_t>> visits;
@@ -192,11 +204,17 @@ struct Model {
   // ws_ldescend over one unit's children [c0, c1)
   struct Worker {
     bool qfull = false;
+    uint32_t iters = 0;
   };
   void walk(uint64_t unit, uint64_t c0, uint64_t c1, Worker& w) {
     uint64_t end = c1;
     bool& qfull = w.qfull;
     for (uint64_t c = c0; c < end; c += 64) {
+      // ws_step
+      const bool beat = step_weight && ws_beat(w.iters, step_weight);
+      w.iters += step_weight;
+      if (beat) ctl.progress.fetch_add(1, std::memory_order_relaxed);
+      if (step_us) std::this_thread::sleep_for(std::chrono::microseconds(step_us));
       if (!qfull && ws_should_split(c, end, split)) {
         const uint64_t k = ws_pieces(c, end, split);
         uint64_t got = 0;
@@ -291,7 +309,8 @@ struct Model {
       if (ctl.busy.load(std::memory_order_relaxed) == 0 &&
           ctl.q_head.load(std::memory_order_relaxed) >= queue_end())
         break;
-      const uint64_t prog = ctl.progress.load(std::memory_order_relaxed);
+      const uint64_t prog = ws_moved(ctl.progress.load(std::memory_order_relaxed),
+                                     ctl.busy.load(std::memory_order_relaxed));
       const uint64_t now = now_ns();
       if (prog != seen) {
         seen = prog;
@@ -335,6 +354,25 @@ static void run_case(uint64_t units, uint64_t split, uint64_t cap, int workers, 
               workers, m.visits.size(), (unsigned long long)m.ctl.pushed.load());
 }
 
+// One unit that takes far longer than the stall limit while every other worker is idle: nothing is
+// wrong as long as its worker's steps report, and the limit is what ends the waits if they do not.
+static void run_slow_unit(bool reports) {
+  Model m(3, 1 << 20, 16, 4, 13, false);
+  for (uint64_t u = 0; u < 3; ++u) {
+    m.width[u] = u == 1 ? 64 * 300 : 64;
+    m.first[u + 1] = m.first[u] + m.width[u];
+  }
+  m.visits = std::vector<std::atomic<uint32_t>>(m.first[3]);
+  m.step_us = 5000;             // 1.5 s in all
+  m.stall_ns = 400'000'000ull;
+  m.step_weight = reports ? kBeatSteps / 8 : 0;  // a report every 40 ms, or none
+  const uint32_t flags = m.run();
+  for (auto& v : m.visits) CHECK(v.load() == 1, "a child of a slow unit visited %u times", v.load());
+  CHECK(flags == (reports ? 0u : 1u), "slow unit %s reports: flags %u", reports ? "with" : "without",
+        flags);
+  std::printf("slow unit %s reports: flag %u\n", reports ? "with" : "without", flags);
+}
+
 int main() {
   check_split_math();
   check_claim_math();
@@ -354,6 +392,8 @@ int main() {
     run_case(u, 0, 16, hw, 20 + u);
     run_case(u, 128, 64, hw, 60 + u);
   }
+  run_slow_unit(true);
+  run_slow_unit(false);
   // a reserved slot whose flag never comes: the taker gives up with the error flag
   Model m(200, 64, 4096, hw, 8, true);
   m.stall_ns = 200'000'000ull;

@@ -8,7 +8,7 @@
 // and writes into chunks in a single pass, falling back to residual passes when chunks run out.
 //
 // Here persistent waves run the frontier DFS of probe_engine.h:
-//   * a wave claims units of 64 probe rows from a global counter, in guided chunks;
+//   * a wave claims units of 64 probe rows from global counters, in guided chunks;
 //   * when a level of its frontier has more than `split` children left, it keeps the next
 //     `split` and publishes the rest as tasks of `split` children each; a task is the 64-lane
 //     frontier of that level (bindings, runs, prefix) plus its child range, so the wave that
@@ -17,7 +17,7 @@
 //     full buffer (not per tuple, nor per last-level frontier);
 //   * a wave leaves when no unit is left, the queue is empty and no wave holds work (a wave
 //     holding work is running, so it finishes and, having pushed tasks, takes them itself if
-//     nobody else does). Every wait is bounded: a wave that sees no unit or task completed
+//     nobody else does). Every wait is bounded: a wave that sees no progress
 //     anywhere for the time limit raises an error flag and leaves, so the kernel always ends.
 // With dro the output is allocated from a sampled estimate before the single pass; if the
 // reservations overrun it, the pass knows the exact total and is run once more into an exact

@@ -285,7 +285,8 @@ constexpr uint32_t stage_ints() {
   return SH == kShapeFour ? kFourTable + kCliqueOther + kPairTable + kQueueWords
                           : kTriTable + kQueueWords;
 }
-static_assert(kStageInts <= kTriTable && kCliqueOther <= kFourTable, "a list fits its table's room");
+static_assert(kStageInts <= kTriTable && kCliqueOther <= kFourTable && kCliqueOther <= kPairTable,
+              "a list fits its table's room");
 static_assert(kStageInts <= kFourTable, "descend_last_fixed stages into the 4-clique's table");
 
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, int lane) {
@@ -499,7 +500,7 @@ constexpr uint32_t kStreamMean = 96;
 // Which of an entry's two child lists is checked against and which is streamed. With lists free of
 // duplicates that are whole (not cut to a window of candidates) the first relation's list is
 // kept in LDS and the second one's streamed: consecutive entries share their first value, so
-// the kept list and its bitmap stay. Otherwise the candidates' own list is streamed, which is what
+// the kept list and its table stay. Otherwise the candidates' own list is streamed, which is what
 // decides how often a duplicate is produced.
 template <int A>
 struct PairLists {
@@ -779,15 +780,7 @@ __device__ __forceinline__ void descend_clique_pairs(const LPlan& P, const LLv<A
     b[0] = (int32_t)readlane_u32((uint32_t)par.b[0], p);
     b[1] = (int32_t)readlane_u32((uint32_t)par.b[1], p);
     const uint64_t h01 = Sink::kHashes ? hash_first_pair<A>(b[0], b[1]) : 0ull;
-    // a list longer than the table's room is searched where it lies
-    if (nl <= kPairTable) {
-      pair.t = lst + kCliqueOther;
-      pair.fill(nl, kPairTable, [&](uint32_t i) { return lst[i]; });
-    } else {
-      pair.t = lst;
-      pair.n = nl;
-      pair.m4 = 0;
-    }
+    pair.fill(nl, kPairTable, [&](uint32_t i) { return lst[i]; });
     // every a2 of L (64 at a time), its children in (2,3) checked against L: streamed list by
     // list, or, when the lists are short, flattened over the wave
     for (uint32_t g0 = 0; g0 < nl; g0 += (uint32_t)kWave) {

@@ -102,10 +102,13 @@ typedef struct {
                                    AMJ_ERR_STATE instead of hanging (0: 20,000 ms); working
                                    waves report progress as they go, so a slow pass is not
                                    mistaken for a stuck one */
-  uint32_t ws_claim_units;      /* ws: most units (64 probe rows or roots each) a wave claims at
-                                   once (0: 64); claims shrink with the remaining units: half
-                                   of them per wave and at least 4 units in launches of 64 or
-                                   more units per wave, else a quarter and at least 1 */
+  uint32_t ws_claim_units;      /* ws: most units a wave claims at once (0: 64; for triangles and
+                                   4-cliques at the default split 1). A unit is 64 probe rows or
+                                   roots (triangles and 4-cliques at the default split: down to
+                                   4 roots, two units per wave). Claims shrink with the
+                                   remaining units: half of them per wave and at least 4 in
+                                   launches of 16 or more units per wave, else a quarter and at
+                                   least 1 */
   uint32_t reserved[2];
 } amj_opts_t;
 #define AMJ_ENGINE_WAVE 0

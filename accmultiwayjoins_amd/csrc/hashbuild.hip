@@ -122,7 +122,7 @@ hipError_t launch_bucket_index(const int32_t* keys, uint64_t n, uint64_t buckets
 
 // The whole build of a table of up to 1024 * ITEMS rows in one workgroup: rows in registers, every
 // sorting pass through one LDS copy, then the columns and the bucket pointers. Bound
-// by the latency of its few passes: 19 us for 4,096 rows, where the tiled build (three kernels per
+// by the latency of its few passes: 16 us for 4,096 rows, where the tiled build (three kernels per
 // digit and three around them) takes about 90. 8,192 rows are what registers and LDS hold at
 // eight rows per lane.
 constexpr int kSmallThreads = 1024;
